@@ -1415,10 +1415,11 @@ static bool attention_short_fits(const AttentionArgs& a) {
   return a.T <= 2 * kKeyTile && a.RP <= 256 && (a.S <= 2 || !(a.flags & kAttnMix));
 }
 
-void launch_routed_attention(const AttentionArgs& a, void* partials, hipStream_t stream) {
+void launch_routed_attention(const AttentionArgs& a, void* scratch, int64_t scratch_bytes, hipStream_t stream) {
   if (a.T == 0 || a.B == 0) return;
+  if (!attention_short_fits(a) && launch_attention_tile(a, scratch, scratch_bytes, stream)) return;
   AttnParams p;
-  p.part = static_cast<char*>(partials);
+  p.part = static_cast<char*>(scratch);
   p.q = a.q;
   p.k = a.k;
   p.qk_stride_b = a.qk_stride_b;
@@ -1450,8 +1451,11 @@ void launch_routed_attention(const AttentionArgs& a, void* partials, hipStream_t
     else launch_attn_short_r<__bf16, __bf16>(a, p, stream);
     return;
   }
-  const AttnPlan plan = plan_attention(a.B, a.S, a.T, a.D, a.RP, (a.flags & kAttnMix) && a.S > 1,
-                                       a.flags & kAttnCausal, partials != nullptr, attn_piece_bytes(a.flags));
+  const bool multi = (a.flags & kAttnMix) && a.S > 1;
+  const int piece_bytes = attn_piece_bytes(a.flags);
+  AttnPlan plan = plan_attention(a.B, a.S, a.T, a.D, a.RP, multi, a.flags & kAttnCausal, scratch != nullptr, piece_bytes);
+  if (plan.part_bytes > scratch_bytes)
+    plan = plan_attention(a.B, a.S, a.T, a.D, a.RP, multi, a.flags & kAttnCausal, false, piece_bytes);
   if (a.qk_dtype == kF16 && a.v_dtype == kBF16) launch_attn_0<_Float16, __bf16>(a, plan, p, stream);
   else if (a.qk_dtype == kF16) launch_attn_0<_Float16, _Float16>(a, plan, p, stream);
   else launch_attn_0<__bf16, __bf16>(a, plan, p, stream);

@@ -284,13 +284,24 @@ int da_dictionary_route_backward_rows(const float* logits, const float* grad_wei
   return check_launch("route backward rows");
 }
 
-int64_t da_attention_workspace_bytes(int64_t batch, int64_t maps, int64_t length, int64_t score_dim,
+// The least workspace a call may pass (when it passes one): the key-range
+// split of the general kernel.
+static int64_t attention_least_bytes(int64_t batch, int64_t maps, int64_t length, int64_t score_dim,
                                      int64_t value_dim, int flags) {
   if (batch < 1 || maps < 1 || length < 1 || value_dim < 1) return 0;
   const bool multi = (flags & DA_ATTN_MIX) && maps > 1;
   return align_up(da::plan_attention(batch, maps, length, value_dim, score_dim, multi, flags & DA_ATTN_CAUSAL, true,
                                      (flags & DA_ATTN_OUT_F32) ? 4 : 2)
                       .part_bytes);
+}
+
+int64_t da_attention_workspace_bytes(int64_t batch, int64_t maps, int64_t length, int64_t score_dim,
+                                     int64_t value_dim, int flags) {
+  if (batch < 1 || maps < 1 || length < 1 || value_dim < 1) return 0;
+  const bool causal = flags & DA_ATTN_CAUSAL;
+  const int es = (flags & DA_ATTN_OUT_F32) ? 4 : 2;
+  const int64_t tile = da::attention_tile_bytes(batch, maps, length, value_dim, score_dim, causal, es);
+  return std::max(attention_least_bytes(batch, maps, length, score_dim, value_dim, flags), align_up(tile));
 }
 
 int da_routed_attention(const void* query, const void* key, int64_t stride_b, int64_t stride_t,
@@ -314,7 +325,7 @@ int da_routed_attention(const void* query, const void* key, int64_t stride_b, in
   // fp32 outputs are written as 16-byte vectors of four floats.
   if ((flags & DA_ATTN_OUT_F32) && !aligned(out, 16))
     return fail(DA_ERR_ALIGNMENT, "attention: fp32 out (DA_ATTN_OUT_F32) must be 16-byte aligned");
-  const int64_t need = da_attention_workspace_bytes(batch, maps, length, score_dim, value_dim, flags);
+  const int64_t need = attention_least_bytes(batch, maps, length, score_dim, value_dim, flags);
   if (workspace && need > 0) {
     if (!aligned(workspace, 256)) return fail(DA_ERR_ALIGNMENT, "attention: workspace must be 256-byte aligned");
     if (workspace_bytes < need)
@@ -349,7 +360,9 @@ int da_routed_attention(const void* query, const void* key, int64_t stride_b, in
   a.out_stride_b = out_stride_b;
   a.out_stride_t = out_stride_t;
   a.out_stride_s = out_stride_s;
-  da::launch_routed_attention(a, need > 0 ? workspace : nullptr, reinterpret_cast<hipStream_t>(stream));
+  const bool usable = workspace && workspace_bytes > 0 && aligned(workspace, 256);
+  da::launch_routed_attention(a, usable ? workspace : nullptr, usable ? workspace_bytes : 0,
+                              reinterpret_cast<hipStream_t>(stream));
   return check_launch("attention");
 }
 
@@ -698,8 +711,9 @@ int64_t da_sda_workspace_offset(int64_t batch, int64_t length, int64_t model_dim
   return routed + vt;
 }
 
-// Split-key partials of the outer attention (one map only: then the score
-// width equals qk_width); the larger of the causal and non-causal plans.
+// Split-key partials of the outer attention's general kernel (one map only:
+// then the score width equals qk_width); the larger of the causal and
+// non-causal plans.
 static int64_t attention_partial_bytes(int64_t batch, int64_t length, int64_t model_dim, int64_t qk_width,
                                        int64_t outer_maps) {
   if (outer_maps != 1) return 0;
@@ -708,13 +722,35 @@ static int64_t attention_partial_bytes(int64_t batch, int64_t length, int64_t mo
   return align_up(std::max(causal.part_bytes, full.part_bytes));
 }
 
+// Scratch of the outer attention in a forward of this shape: the general
+// kernel's partials or the eight-wave kernel's.
+static int64_t attention_scratch_bytes(int64_t batch, int64_t length, int64_t model_dim, int64_t qk_width,
+                                       int64_t outer_maps) {
+  int64_t tile = 0;
+  for (const bool causal : {false, true})
+    tile = std::max(tile, da::attention_tile_bytes(batch, outer_maps, length, model_dim, qk_width, causal, 2));
+  return std::max(attention_partial_bytes(batch, length, model_dim, qk_width, outer_maps), align_up(tile));
+}
+
+static int64_t sda_mixed_bytes(int64_t tokens, int64_t model_dim, int64_t outer_maps, bool concat, bool projected) {
+  return projected ? align_up(tokens * (concat ? outer_maps : 1) * model_dim * 2) : 0;
+}
+
+// The least workspace a forward accepts: with less than da_sda_workspace_bytes
+// the outer attention takes its general kernel.
+static int64_t sda_least_bytes(int64_t batch, int64_t length, int64_t model_dim, int64_t qk_width,
+                               int64_t outer_maps, bool concat, bool projected) {
+  return da_sda_workspace_offset(batch, length, model_dim, qk_width, 2) +
+         sda_mixed_bytes(batch * length, model_dim, outer_maps, concat, projected) +
+         attention_partial_bytes(batch, length, model_dim, qk_width, outer_maps);
+}
+
 int64_t da_sda_workspace_bytes(int64_t batch, int64_t length, int64_t model_dim, int64_t qk_width,
                                int64_t outer_maps, int concat, int has_output_projection) {
-  const int64_t tokens = batch * length;
-  const int64_t mixed =
-      has_output_projection ? align_up(tokens * (concat ? outer_maps : 1) * model_dim * 2) : 0;
-  return da_sda_workspace_offset(batch, length, model_dim, qk_width, 2) + mixed +
-         attention_partial_bytes(batch, length, model_dim, qk_width, outer_maps);
+  if (outer_maps < 1) return 0;
+  return da_sda_workspace_offset(batch, length, model_dim, qk_width, 2) +
+         sda_mixed_bytes(batch * length, model_dim, outer_maps, concat != 0, has_output_projection != 0) +
+         attention_scratch_bytes(batch, length, model_dim, qk_width, outer_maps);
 }
 
 int da_shared_dictionary_attention_forward(const da_sda_forward_args* a, da_stream_t stream) {
@@ -732,7 +768,7 @@ int da_shared_dictionary_attention_forward(const da_sda_forward_args* a, da_stre
   const bool concat = a->flags & DA_SDA_CONCAT;
   if (concat && !a->wo) return fail(DA_ERR_INVALID_ARGUMENT, "forward: concat combine needs an output projection");
   if (!aligned(a->workspace, 256)) return fail(DA_ERR_ALIGNMENT, "forward: workspace must be 256-byte aligned");
-  const int64_t need = da_sda_workspace_bytes(B, T, d, H * R, S, concat, a->wo != nullptr);
+  const int64_t need = sda_least_bytes(B, T, d, H * R, S, concat, a->wo != nullptr);
   if (a->workspace_bytes < need)
     return fail(DA_ERR_WORKSPACE, "forward: workspace of %lld bytes < %lld required",
                 (long long)a->workspace_bytes, (long long)need);
@@ -744,10 +780,12 @@ int da_shared_dictionary_attention_forward(const da_sda_forward_args* a, da_stre
   void* routed = ws;
   void* vt = ws + da_sda_workspace_offset(B, T, d, W, 1);
   void* mixed = a->wo ? ws + da_sda_workspace_offset(B, T, d, W, 2) : a->out;
-  const int64_t mixed_bytes = a->wo ? align_up(B * T * (concat ? S : 1) * d * 2) : 0;
-  void* partials = attention_partial_bytes(B, T, d, W, S) > 0
-                       ? ws + da_sda_workspace_offset(B, T, d, W, 2) + mixed_bytes
-                       : nullptr;
+  // What follows in the workspace is the outer attention's scratch (the same
+  // share whatever else the caller's buffer holds).
+  const int64_t scratch_at =
+      da_sda_workspace_offset(B, T, d, W, 2) + sda_mixed_bytes(B * T, d, S, concat, a->wo != nullptr);
+  const int64_t scratch_bytes =
+      std::min(a->workspace_bytes - scratch_at, attention_scratch_bytes(B, T, d, W, S));
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
 
   // Validate every stage before enqueueing the first one.
@@ -844,7 +882,7 @@ int da_shared_dictionary_attention_forward(const da_sda_forward_args* a, da_stre
   at.out_stride_b = T * ot;
   at.out_stride_t = ot;
   at.out_stride_s = concat ? d : 0;
-  da::launch_routed_attention(at, partials, s);
+  da::launch_routed_attention(at, scratch_bytes > 0 ? ws + scratch_at : nullptr, scratch_bytes, s);
   // 4. Output projection.
   if (a->wo) {
     da::GemmSegment o{a->wo, nullptr, 0, mixed, d, B * T, ot, nullptr, 0, 0, a->out, d, 0, 0, 0, da::kGemmActNone,
@@ -906,9 +944,9 @@ extern "C" int da_shared_dictionary_attention_forward_noalloc(const da_sda_forwa
   if (args->batch < 1 || args->length < 1 || args->model_dim < 1 || args->qk_branches < 1 || args->routing_dim < 1 ||
       args->outer_maps < 1)
     return fail(DA_ERR_INVALID_ARGUMENT, "noalloc forward: sizes must be positive");
-  const int64_t need = da_sda_workspace_bytes(args->batch, args->length, args->model_dim,
-                                              args->qk_branches * args->routing_dim, args->outer_maps,
-                                              (args->flags & DA_SDA_CONCAT) != 0, args->wo != nullptr);
+  const int64_t need = sda_least_bytes(args->batch, args->length, args->model_dim,
+                                       args->qk_branches * args->routing_dim, args->outer_maps,
+                                       (args->flags & DA_SDA_CONCAT) != 0, args->wo != nullptr);
   if (need > DA_NOALLOC_SCRATCH_BYTES)
     return fail(DA_ERR_WORKSPACE,
                 "noalloc forward: the problem needs %lld bytes of scratch, more than the %lld-byte per-GPU array "

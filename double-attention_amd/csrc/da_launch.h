@@ -272,9 +272,16 @@ struct AttnPlan {
 };
 AttnPlan plan_attention(int64_t B, int64_t S, int64_t T, int64_t D, int64_t RP, bool multi, bool causal,
                         bool allow_split, int piece_bytes);
-// `partials`: plan.part_bytes of device scratch (plan with allow_split), or
-// nullptr to run without key-range splitting.
-void launch_routed_attention(const AttentionArgs& a, void* partials, hipStream_t stream);
+// `scratch`: device scratch of the call, or nullptr.  A kernel or split that
+// needs more than scratch_bytes is not taken.
+void launch_routed_attention(const AttentionArgs& a, void* scratch, int64_t scratch_bytes, hipStream_t stream);
+// The eight-wave kernel (attention_tile.hip): fp16 queries and keys, one map
+// over a long sequence.  Scratch bytes of a call with outputs of es bytes (0:
+// none, or not taken), and the launch itself: false when the call is not one
+// it takes, or needs more scratch than it is given.
+int64_t attention_tile_bytes(int64_t B, int64_t S, int64_t T, int64_t D, int64_t RP, bool causal, int es);
+bool launch_attention_tile(const AttentionArgs& a, void* workspace, int64_t workspace_bytes, hipStream_t stream);
+
 struct NormJob;
 // `norm`: a dictionary normalization run by extra workgroups of the same
 // launch, or nullptr.

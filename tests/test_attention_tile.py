@@ -1,0 +1,91 @@
+"""The eight-wave attention kernel.
+
+Calls the C entry point at the sizes where the tiling can go wrong (edges of
+the 128-query and 32-key tiles, split and whole key ranges, one and two
+value slices), against the NumPy oracle.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from double_attention import _lib
+
+pytestmark = pytest.mark.gpu
+
+F16, BF16 = _lib.DA_F16, _lib.DA_BF16
+
+
+def _case(batch, maps, length, score_dim, value_dim, dtype, causal, log_scale, bound, out_f32=False):
+    g = torch.Generator().manual_seed(length + score_dim)
+    rows = torch.nn.functional.normalize(torch.randn(batch, length, 2, maps, score_dim, generator=g), dim=-1).half()
+    value = torch.randn(batch, length, value_dim, generator=g).to(dtype)
+    scales = torch.linspace(log_scale - 0.4, log_scale + 0.4, maps) if maps > 1 else torch.tensor([log_scale])
+    logits = torch.linspace(-0.7, 0.9, maps)
+    padded = (length + 63) // 64 * 64
+    tiles = torch.zeros(batch, padded // 32, value_dim, 32, dtype=dtype)
+    full = torch.zeros(batch, padded, value_dim, dtype=dtype)
+    full[:, :length] = value
+    tiles.copy_(full.view(batch, padded // 32, 32, value_dim).transpose(2, 3))
+
+    d = torch.device("cuda:0")
+    rd, td, sd, ld = rows.to(d), tiles.to(d), scales.to(d), logits.to(d)
+    out_dtype = torch.float32 if out_f32 else dtype
+    out = torch.full((batch, length, value_dim), float("nan"), dtype=out_dtype, device=d)
+    flags = _lib.DA_ATTN_SCALES_ARE_LOG | (_lib.DA_ATTN_CAUSAL if causal else 0)
+    flags |= (_lib.DA_ATTN_MIX if maps > 1 else 0) | (_lib.DA_ATTN_OUT_F32 if out_f32 else 0)
+    lib = _lib.get()
+    need = lib.da_attention_workspace_bytes(batch, maps, length, score_dim, value_dim, flags)
+    workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=d)
+    width = maps * score_dim
+
+    def call(nbytes):
+        out.fill_(float("nan"))
+        _lib.check(
+            lib.da_routed_attention(
+                rd.data_ptr(), rd.data_ptr() + width * 2, length * 2 * width, 2 * width, score_dim, 1, score_dim,
+                td.data_ptr(), td.stride(0), batch, maps, length, value_dim, sd.data_ptr(), _lib.DA_F32, 1.0,
+                ld.data_ptr() if maps > 1 else None, _lib.DA_F32, flags, bound,
+                F16, BF16 if dtype == torch.bfloat16 else F16, out.data_ptr(), out.stride(0), out.stride(1), 0,
+                workspace.data_ptr() if nbytes else None, nbytes, torch.cuda.current_stream().cuda_stream,
+            ),
+            "attention",
+        )
+        torch.cuda.synchronize()
+        return out.float().cpu().numpy()
+
+    q, k = (rows[:, :, i].permute(0, 2, 1, 3).float().numpy() for i in (0, 1))
+    per_map = oracle.routed_attention(q, k, value.float().numpy(), np.exp(scales.numpy()), causal)
+    alpha = torch.softmax(logits, 0).numpy() if maps > 1 else np.ones(1, np.float32)
+    return call, need, np.einsum("s,bstd->btd", alpha, per_map)
+
+
+@pytest.mark.parametrize("case", [
+    # batch, maps, length, score width, value width, dtype, causal, log scale, bound, fp32 out
+    (1, 1, 2048, 256, 512, torch.bfloat16, True, 2.77, 1.01, False),
+    (1, 1, 2081, 256, 512, torch.bfloat16, True, 2.77, 1.01, True),      # ragged last tiles, fp32 pieces
+    (1, 1, 2111, 256, 768, torch.float16, True, 2.77, 1.01, False),      # row maxima first, three 256-wide slices
+    (1, 1, 2049, 256, 256, torch.bfloat16, False, 6.0, 1.01, False),     # scale past the fixed reference
+    (1, 1, 2177, 256, 512, torch.bfloat16, False, 2.77, 1.01, False),    # split without a mask
+    (1, 1, 1024, 512, 512, torch.bfloat16, True, 3.1, 1.01, False),
+    (2, 1, 1055, 512, 256, torch.float16, True, 3.1, 0.0, True),         # no bound
+    (9, 1, 1024, 512, 256, torch.bfloat16, False, 3.1, 1.01, False),     # whole key ranges
+])
+def test_attention_tile(case) -> None:
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    print(f"[attention tile] {case}", flush=True)
+    call, need, expected = _case(*case)
+    assert need > 0 or case[0] == 9
+    got = call(need)
+    # One 16-bit rounding of P, V and the output each, averaged over the keys:
+    # well under the operand type's half unit in the last place.
+    bar = 5e-3 if case[5] == torch.bfloat16 else 1e-3
+    rel = np.linalg.norm(got - expected) / np.linalg.norm(expected)
+    assert np.isfinite(got).all() and rel <= bar, rel
+    # Without scratch the general kernel takes the call.
+    general = call(0)
+    assert np.linalg.norm(general - got) / np.linalg.norm(expected) <= 2 * bar
