@@ -71,18 +71,21 @@ __device__ __forceinline__ float dbeta_at(int flags, float dbeta, float beta_raw
 }
 
 // WPR waves per row: with WPR = 1 a workgroup's four waves take four rows;
-// with WPR = 4 its waves share one row (column j at wave j / 64 % 4), and the
-// row sums meet in LDS.
-template <typename TO, int NPL, int WPR>
+// with WPR = 4 its waves share one row, and the row sums meet in LDS.  A lane
+// holds NPL / VEC runs of VEC columns; VAR builds the variants in (without
+// them c is l, and fewer registers keep more rows in flight).
+template <typename TO, int NPL, int WPR, int VEC, bool VAR>
 __global__ __launch_bounds__(256) void route_backward_rows_kernel(RouteBwdRowsArgs a) {
   static_assert(WPR == 1 || WPR == 4, "one wave per row, or the workgroup's four");
-  constexpr int STRIDE = 64 * WPR;   // columns between a lane's consecutive elements
+  static_assert((VEC == 1 || VEC == 4) && NPL % VEC == 0, "single columns or 16-byte runs");
+  constexpr int STRIDE = 64 * WPR * VEC;   // columns between a lane's consecutive runs
   __shared__ float red[2][WPR];
   const int lane = lane_id();
   const int wave = uniform_wave();
   const int64_t row = WPR == 1 ? static_cast<int64_t>(blockIdx.x) * 4 + wave : static_cast<int64_t>(blockIdx.x);
   if (row >= a.rows) return;   // whole waves (WPR 1), or the whole workgroup
-  const int col0 = (WPR == 1 ? 0 : wave * 64) + lane;
+  const int col0 = ((WPR == 1 ? 0 : wave * 64) + lane) * VEC;
+  auto col = [&](int i) { return col0 + STRIDE * (i / VEC) + i % VEC; };
   // Sum or maximum over the row: the wave's lanes, then (WPR 4) the four
   // waves through one of two LDS slots in turn, so one barrier per call.
   int slot = 0;
@@ -103,20 +106,39 @@ __global__ __launch_bounds__(256) void route_backward_rows_kernel(RouteBwdRowsAr
   const int M = a.causal_period ? min(a.atoms, static_cast<int>(row % a.causal_period) + 1) : a.atoms;
   const float* lrow = a.logits + row * a.ld_in;
   const float* grow = a.grad_weights + row * a.ld_in;
-  const bool silu_logits = a.flags & kRouteSiluLogits;
-  const bool standardize = a.flags & kRouteStandardize;
-  const bool direct = a.flags & kRouteDirectSilu;
+  const bool silu_logits = VAR && (a.flags & kRouteSiluLogits);
+  const bool standardize = VAR && (a.flags & kRouteStandardize);
+  const bool direct = VAR && (a.flags & kRouteDirectSilu);
 
   // beta of this row: one value, or entry (row / beta_period) % beta_count.
   const int64_t beta_index = a.beta_count > 1 ? (row / a.beta_period) % a.beta_count : 0;
   const ScalarHalves beta_bits = fetch_scalar(a.beta_ptr ? a.beta_ptr : static_cast<const void*>(a.logits),
                                               a.beta_ptr ? a.beta_dtype : kF32, a.beta_ptr ? beta_index : 0);
+  // Columns past M re-read the row's last run (a load under a condition would
+  // wait for its data at the end of the branch) and count as zero.
   float l[NPL], g[NPL];
+  const int last = (M - 1) / VEC * VEC;
+#pragma unroll
+  for (int i = 0; i < NPL; i += VEC) {
+    const int j = min(col(i), last);
+    if constexpr (VEC == 4) {
+      const f32x4 lv = *reinterpret_cast<const f32x4*>(lrow + j);
+      const f32x4 gv = *reinterpret_cast<const f32x4*>(grow + j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        l[i + e] = lv[e];
+        g[i + e] = gv[e];
+      }
+    } else {
+      l[i] = lrow[j];
+      g[i] = grow[j];
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int i = 0; i < NPL; ++i) {
-    const int j = col0 + STRIDE * i;
-    l[i] = j < M ? lrow[j] : 0.f;
-    g[i] = j < M ? grow[j] : 0.f;
+    l[i] = col(i) < M ? l[i] : 0.f;
+    g[i] = col(i) < M ? g[i] : 0.f;
   }
   const float beta_raw = a.beta_ptr ? scalar_value(beta_bits, a.beta_dtype) : a.beta_value;
   const float beta = beta_from(a.flags, beta_raw);
@@ -131,12 +153,12 @@ __global__ __launch_bounds__(256) void route_backward_rows_kernel(RouteBwdRowsAr
   if (standardize) {
     float s1 = 0.f;
 #pragma unroll
-    for (int i = 0; i < NPL; ++i) s1 += col0 + STRIDE * i < M ? c[i] : 0.f;
+    for (int i = 0; i < NPL; ++i) s1 += col(i) < M ? c[i] : 0.f;
     const float mean = row_reduce(s1, false) * inv_m;
     float s2 = 0.f;
 #pragma unroll
     for (int i = 0; i < NPL; ++i) {
-      c[i] = col0 + STRIDE * i < M ? c[i] - mean : 0.f;
+      c[i] = col(i) < M ? c[i] - mean : 0.f;
       s2 += c[i] * c[i];
     }
     isd = rsqrtf(row_reduce(s2, false) * inv_m + a.eps);
@@ -159,12 +181,12 @@ __global__ __launch_bounds__(256) void route_backward_rows_kernel(RouteBwdRowsAr
     float mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < NPL; ++i)
-      if (col0 + STRIDE * i < M) mx = fmaxf(mx, beta * (c[i] * s));
+      if (col(i) < M) mx = fmaxf(mx, beta * (c[i] * s));
     mx = row_reduce(mx, true);
     float z = 0.f;
 #pragma unroll
     for (int i = 0; i < NPL; ++i) {
-      w[i] = col0 + STRIDE * i < M ? __expf(beta * (c[i] * s) - mx) : 0.f;
+      w[i] = col(i) < M ? __expf(beta * (c[i] * s) - mx) : 0.f;
       z += w[i];
     }
     const float inv_z = 1.f / row_reduce(z, false);
@@ -207,9 +229,19 @@ __global__ __launch_bounds__(256) void route_backward_rows_kernel(RouteBwdRowsAr
   TO* dl_row = static_cast<TO*>(a.grad_logits) + row * a.ld_out;
   TO* w_row = static_cast<TO*>(a.weights) + row * a.ld_out;
 #pragma unroll
-  for (int i = 0; i < NPL; ++i) {
-    const int j = col0 + STRIDE * i;
-    if (j < a.atoms) {
+  for (int i = 0; i < NPL; i += VEC) {
+    const int j = col(i);
+    if (j >= a.atoms) continue;
+    if constexpr (VEC == 4) {
+      typename Elem<TO>::v4 dv, wv;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        dv[e] = static_cast<TO>(j + e < M ? g[i + e] : 0.f);
+        wv[e] = static_cast<TO>(j + e < M ? w[i + e] : 0.f);
+      }
+      *reinterpret_cast<typename Elem<TO>::v4*>(dl_row + j) = dv;
+      *reinterpret_cast<typename Elem<TO>::v4*>(w_row + j) = wv;
+    } else {
       dl_row[j] = static_cast<TO>(j < M ? g[i] : 0.f);
       w_row[j] = static_cast<TO>(j < M ? w[i] : 0.f);
     }
@@ -390,26 +422,41 @@ __global__ __launch_bounds__(256) void route_backward_long_rows_kernel(RouteBwdR
   if (a.dbeta_rows && lane == 0) a.dbeta_rows[row] = direct ? 0.f : dbeta_at(a.flags, dbeta, beta_raw, beta);
 }
 
+template <typename TO, int NPL, int WPR>
+static void launch_route_bwd_rows_n(const RouteBwdRowsArgs& a, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(WPR == 1 ? (a.rows + 3) / 4 : a.rows));
+  // Runs of four columns need whole, aligned 16-byte loads and 8-byte stores.
+  const auto at = [](const void* p, int bytes) { return reinterpret_cast<uintptr_t>(p) % bytes == 0; };
+  const bool runs = a.atoms % 4 == 0 && a.ld_in % 4 == 0 && a.ld_out % 4 == 0 && at(a.logits, 16) &&
+                    at(a.grad_weights, 16) && at(a.grad_logits, 8) && at(a.weights, 8);
+  if (a.flags & kRouteVariants) {
+    if (runs) hipLaunchKernelGGL((route_backward_rows_kernel<TO, NPL, WPR, 4, true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((route_backward_rows_kernel<TO, NPL, WPR, 1, true>), grid, dim3(256), 0, s, a);
+  } else {
+    if (runs) hipLaunchKernelGGL((route_backward_rows_kernel<TO, NPL, WPR, 4, false>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((route_backward_rows_kernel<TO, NPL, WPR, 1, false>), grid, dim3(256), 0, s, a);
+  }
+}
+
 template <typename TO>
 static void launch_route_bwd_rows_t(const RouteBwdRowsArgs& a, hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>((a.rows + 3) / 4));
   // Up to 4096 columns one wave holds a row; up to 16384 the workgroup's four
   // waves share it (32 or 64 columns per lane); longer rows take passes.
-  const dim3 per_row(static_cast<unsigned>(a.rows));
   if (a.atoms > 16384) {
+    const dim3 grid(static_cast<unsigned>((a.rows + 3) / 4));
     hipLaunchKernelGGL((route_backward_long_rows_kernel<TO>), grid, dim3(256), 0, s, a);
   } else if (a.atoms > 8192) {
-    hipLaunchKernelGGL((route_backward_rows_kernel<TO, 64, 4>), per_row, dim3(256), 0, s, a);
+    launch_route_bwd_rows_n<TO, 64, 4>(a, s);
   } else if (a.atoms > 4096) {
-    hipLaunchKernelGGL((route_backward_rows_kernel<TO, 32, 4>), per_row, dim3(256), 0, s, a);
+    launch_route_bwd_rows_n<TO, 32, 4>(a, s);
   } else if (a.atoms <= 512) {
-    hipLaunchKernelGGL((route_backward_rows_kernel<TO, 8, 1>), grid, dim3(256), 0, s, a);
+    launch_route_bwd_rows_n<TO, 8, 1>(a, s);
   } else if (a.atoms <= 1024) {
-    hipLaunchKernelGGL((route_backward_rows_kernel<TO, 16, 1>), grid, dim3(256), 0, s, a);
+    launch_route_bwd_rows_n<TO, 16, 1>(a, s);
   } else if (a.atoms <= 2048) {
-    hipLaunchKernelGGL((route_backward_rows_kernel<TO, 32, 1>), grid, dim3(256), 0, s, a);
+    launch_route_bwd_rows_n<TO, 32, 1>(a, s);
   } else {
-    hipLaunchKernelGGL((route_backward_rows_kernel<TO, 64, 1>), grid, dim3(256), 0, s, a);
+    launch_route_bwd_rows_n<TO, 64, 1>(a, s);
   }
 }
 
