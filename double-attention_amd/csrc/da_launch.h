@@ -29,6 +29,11 @@ enum : int {
                                 // outer attention's temperature (clamp window
                                 // kLogScaleMin .. kLogScaleMax)
 };
+// The flags that change how logits become weights.
+constexpr int kRouteVariants = kRouteSiluLogits | kRouteStandardize | kRouteDirectSilu;
+// Fixed-reference mode keeps the route's fp16 probabilities in
+// [2^(kRouteP16Lift - 2*beta*log2e), 2^kRouteP16Lift].
+constexpr float kRouteP16Lift = 14.f;
 
 // Attention flags.
 enum : int {
@@ -158,6 +163,8 @@ void launch_dictionary_normalize(const void* raw_key, const void* raw_value, int
                                  int M, float eps, void* key_t, int key_dtype, void* value,
                                  void* value_rows, hipStream_t stream);
 void launch_dictionary_route(const RouteArgs& a, hipStream_t stream);
+// 256- or 512-wide rows without kRouteVariants.
+void launch_route_tile(const RouteArgs& a, hipStream_t stream);
 // Backward of the column normalization (dict_norm.hip).  Banks [R, M]
 // row-major of one dtype; gradients fp32 [R, M]; raw_value NULL = tied bank
 // (the key gradient plus grad_value, when given, flows into d_key).

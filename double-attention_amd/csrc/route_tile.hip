@@ -1,0 +1,419 @@
+// Fused dictionary route for 512-wide rows and for few 256-wide ones (plain
+// softmax assignment; route.hip has the contract, the variants, the other rows
+// and the rule between them).
+//
+// A workgroup of eight waves owns QT rows and streams the whole dictionary
+// past them, KT atoms per step:
+//   S^T[j, c] = Dk^T U^T   the step's 16 x 16 blocks are dealt to the waves:
+//       each holds its unit rows in VGPRs and reads its key atoms from LDS;
+//   P^T                    packed as MFMA B operands (da_common.h) into LDS;
+//   O^T[r, c] += Dv P^T    each wave owns R/8 coordinates of all QT rows: it
+//       reads P from LDS and its value atoms straight from memory (the
+//       32-atom tiles make a wave's 16 coordinates one contiguous KiB, and no
+//       other wave of the workgroup needs them).
+// Against four 16-row waves that each read every key and value fragment from
+// LDS (256 KiB per 32 atoms of 64 rows at R = 512), this reads 160 KiB, and two
+// waves share a SIMD.  What bounds it: the chain of one step (key loads, key
+// fragments, exponentials, the P exchange, the barrier), about 3000 clocks for
+// 1024 of MFMA work at R = 512.  A third key buffer with loads a whole step
+// ahead was slower (80 us against 71 at 16384 rows x 1536 atoms).  Measured (us,
+// bf16 rows, beta 8, against route.hip's kernel): R = 512 with 1536 atoms 192 rows 39 /
+// 67, 8192 rows 45 / 70, 16384 rows 62 / 74, 65536 rows 246 / 279; R = 256 with
+// 512 atoms 192 rows 11.0 / 12.9, 8192 rows 12.6 / 14.8, 12000 rows 19.3 / 26.3.
+// Where beta is too large for the fixed reference the extra pass over the
+// logits takes back the gain at 1536 atoms (beta 20: R = 256 8192 rows 33.9 / 32.6,
+// R = 512 8192 rows 61 / 86, 16384 rows 89 / 88).
+// Step t multiplies P(t) while it forms the weights of t+1, one barrier per
+// step; key tiles reach a two-buffer LDS ring by global->LDS DMA issued at the
+// start of a step.
+#include <type_traits>
+
+#include "da_common.h"
+#include "da_launch.h"
+#include "da_tile.h"
+
+namespace da {
+
+namespace {
+
+constexpr int kWaves = 8;
+
+struct RouteTileParams {
+  const void* x;
+  int64_t rows, x_stride;
+  const void* key_t;
+  const _Float16* value;
+  int M, n_tiles;
+  const void* beta_ptr;
+  int beta_dtype;
+  float beta_value, eps;
+  int flags;
+  void* out;
+  int64_t out_stride;
+};
+
+}  // namespace
+
+// QPW: row blocks (of 16) of a wave's score blocks; every key fragment read
+// feeds QPW MFMAs.
+template <typename TX, typename TK, typename TO, int R, int QT, int KT, int QPW>
+__global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams p) {
+  // x and out may alias (in-place routing): the workgroup has read its rows
+  // into VGPRs, a barrier or more before any of its waves writes one.
+  typedef typename Elem<TK>::v8 k8;
+  constexpr int QB = QT / 16;                  // row blocks
+  constexpr int KW = KT / 32;                  // 32-atom windows of a step
+  constexpr int NKG = KT / 16;                 // waves along the atoms, one 16-atom block each
+  static_assert(NKG * (QB / QPW) == kWaves, "the score blocks go round the waves");
+  constexpr int KS = R / 32;
+  constexpr int FB = R / 128;                  // 16-coordinate blocks per wave
+  typedef XorTile<KT, R / 8, true> KTile;
+  constexpr int KCH = KTile::LOADS / kWaves;   // wave loads of a key tile per wave
+  constexpr int PBYTES = KW * QB * 1024;
+  constexpr int OFF_P = 2 * KTile::BYTES;
+  // The P buffers also take the exchanges of row maxima, sums and norms.
+  static_assert(NKG * QT * 4 <= PBYTES && kWaves * QT * 4 <= PBYTES, "the exchanges fit a P buffer each");
+  __shared__ __attribute__((aligned(1024))) char lds[OFF_P + 2 * PBYTES];
+
+  const int lane = lane_id();
+  const int c = lane & 15, g = lane >> 4;
+  const int wave = uniform_wave();
+  const int kg = wave % NKG, qg = wave / NKG;   // this wave's score blocks
+  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * QT;
+  const TX* x = static_cast<const TX*>(p.x);
+
+  // One memory round trip: beta, the rows (past the end the last one repeats,
+  // never stored) and the first key tiles.
+  const ScalarHalves beta_bits = fetch_scalar(p.beta_ptr ? p.beta_ptr : p.x, p.beta_ptr ? p.beta_dtype : kF32, 0);
+  typename Elem<TX>::v8 xr[QPW][KS];
+#pragma unroll
+  for (int i = 0; i < QPW; ++i) {
+    const int64_t left = p.rows - 1 - row0;
+    const int at = (qg * QPW + i) * 16 + c;
+    const TX* src = x + (row0 + (at < left ? at : left)) * p.x_stride + 8 * g;
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) xr[i][kk] = load8(src + kk * 32);
+  }
+  uint32_t koff[KCH];
+#pragma unroll
+  for (int i = 0; i < KCH; ++i) {
+    int row, ck;
+    KTile::slot_chunk((i * kWaves + wave) * 64 + lane, row, ck);
+    koff[i] = static_cast<uint32_t>((row * R + ck * 8) * 2);
+  }
+  // Key atoms of tile t into its buffer (the parity of t); the bank is padded
+  // to whole tiles.
+  auto load_keys = [&](int t) {
+    const char* src = uniform_ptr(static_cast<const char*>(p.key_t) + static_cast<int64_t>(t) * KT * R * 2);
+    char* dst = lds + (t & 1) * KTile::BYTES + wave * 1024;
+#pragma unroll
+    for (int i = 0; i < KCH; ++i) dma16(src + koff[i], dst + i * kWaves * 1024);
+  };
+  const int n_tiles = p.n_tiles;
+  load_keys(0);
+  if (n_tiles > 1) load_keys(1);
+  // Nothing that uses a loaded value moves above the loads' issue.
+  __builtin_amdgcn_sched_barrier(0);
+  wait_vmem();
+
+  const float beta_raw = p.beta_ptr ? scalar_value(beta_bits, p.beta_dtype) : p.beta_value;
+  const float beta = (p.flags & kRouteBetaIsLog) ? expf(fminf(fmaxf(beta_raw, kLogBetaMin), kLogBetaMax)) : beta_raw;
+  // Maxima are taken of raw logits, so a negative beta is folded into the rows.
+  const float scale = fabsf(beta) * kLog2e;
+  const float sign = beta < 0.f ? -1.f : 1.f;
+  // With input normalization the unit row is rounded once to TK; otherwise
+  // TK == TX and the raw row passes through unchanged.
+  k8 xf[QPW][KS];
+#pragma unroll
+  for (int i = 0; i < QPW; ++i) {
+    float ss = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = static_cast<float>(xr[i][kk][e]);
+        ss += v * v;
+      }
+    ss = group_sum(ss);
+    const float inv = sign * ((p.flags & kRouteNormalizeInput) ? 1.f / fmaxf(sqrtf(ss), p.eps) : 1.f);
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xf[i][kk][e] = static_cast<TK>(static_cast<float>(xr[i][kk][e]) * inv);
+  }
+
+  const _Float16* vbase = p.value + 32 * (wave * FB * 16) + c * 32 + g * 8;
+  f16x8 vreg[KW][FB];
+  auto load_values = [&](int t) {
+    const _Float16* src = vbase + static_cast<int64_t>(t) * KT * R;
+#pragma unroll
+    for (int w = 0; w < KW; ++w)
+#pragma unroll
+      for (int f = 0; f < FB; ++f) vreg[w][f] = load8(src + w * 32 * R + f * 16 * 32);
+  };
+
+  int kfrag[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) kfrag[k] = KTile::base(c, g, k) + kg * KTile::ROW_BLOCK;
+  // Logits of tile t: lane (c, g) element e of block i is atom atom_of(t) + e
+  // for row 16 (qg QPW + i) + c.
+  auto logits = [&](int t, f32x4 (&st)[QPW]) {
+    const char* tile = lds + (t & 1) * KTile::BYTES;
+#pragma unroll
+    for (int i = 0; i < QPW; ++i) st[i] = zero4();
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) {
+      const k8 a = lds_v8<TK>(tile + kfrag[kk & 3] + 256 * (kk >> 2));
+#pragma unroll
+      for (int i = 0; i < QPW; ++i) st[i] = Elem<TK>::mma(a, xf[i][kk], st[i]);
+    }
+    // Four fragments stay in flight ahead of their MFMAs.
+    constexpr int AHEAD = 4;
+    __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+    for (int n = 0; n < KS - AHEAD; ++n) {
+      __builtin_amdgcn_sched_group_barrier(0x008, QPW, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, AHEAD * QPW, 0);
+  };
+  auto atom_of = [&](int t) { return t * KT + 32 * (kg >> 1) + 8 * g + 4 * (kg & 1); };
+
+  // The reference of the exponents: fixed where unit rows and unit atoms bound
+  // every logit by 1 and all weights then stay in fp16's normal range, else
+  // each row's maximum from a pass over the atoms.  The largest weight is at
+  // most 2^kRouteP16Lift; the factor cancels in the division by the row sum.
+  const bool fixed = (p.flags & kRouteNormalizeInput) && (p.flags & kRouteUnitKeys) && 2.f * scale <= 2.f * kRouteP16Lift;
+  float ref[QPW];
+#pragma unroll
+  for (int i = 0; i < QPW; ++i) ref[i] = kRouteP16Lift - scale;
+  if (!fixed) {
+    float mx[QPW];
+#pragma unroll
+    for (int i = 0; i < QPW; ++i) mx[i] = -INFINITY;
+    for (int t = 0; t < n_tiles; ++t) {
+      wait_vmem();
+      lds_barrier();
+      if (t > 0 && t + 1 < n_tiles) load_keys(t + 1);
+      f32x4 st[QPW];
+      logits(t, st);
+#pragma unroll
+      for (int i = 0; i < QPW; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (atom_of(t) + e < p.M) mx[i] = fmaxf(mx[i], st[i][e] * scale);
+    }
+    float* xch = reinterpret_cast<float*>(lds + OFF_P);
+#pragma unroll
+    for (int i = 0; i < QPW; ++i) {
+      const float m = group_max(mx[i]);
+      if (g == 0) xch[kg * QT + (qg * QPW + i) * 16 + c] = m;
+    }
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < QPW; ++i) {
+      float m = -INFINITY;
+#pragma unroll
+      for (int w = 0; w < NKG; ++w) m = fmaxf(m, xch[w * QT + (qg * QPW + i) * 16 + c]);
+      ref[i] = m == -INFINITY ? 0.f : kRouteP16Lift - m;
+    }
+    // The pipeline restarts at the first tile (every wave is past its reads of
+    // both key buffers; the barrier below is past the exchange's).
+    wait_vmem();
+    load_keys(0);
+    if (n_tiles > 1) load_keys(1);
+    wait_vmem();
+  }
+
+  f32x4 acc[FB][QB];
+#pragma unroll
+  for (int f = 0; f < FB; ++f)
+#pragma unroll
+    for (int i = 0; i < QB; ++i) acc[f][i] = zero4();
+  float l_part[QPW];
+#pragma unroll
+  for (int i = 0; i < QPW; ++i) l_part[i] = 0.f;
+
+  // Logits of tile t, turned into weights in its P buffer.
+  auto weights = [&](int t) {
+    char* dst = lds + OFF_P + (t & 1) * PBYTES + (kg >> 1) * QB * 1024 + (kg & 1) * 8;
+    f32x4 pr[QPW];
+    logits(t, pr);
+#pragma unroll
+    for (int i = 0; i < QPW; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pr[i][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(pr[i][e], scale, ref[i]));
+    if ((t + 1) * KT > p.M) {   // padding atoms weigh nothing
+#pragma unroll
+      for (int i = 0; i < QPW; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (atom_of(t) + e >= p.M) pr[i][e] = 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < QPW; ++i) {
+      l_part[i] += (pr[i][0] + pr[i][1]) + (pr[i][2] + pr[i][3]);
+      f16x4 h;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) h[e] = static_cast<_Float16>(pr[i][e]);
+      *reinterpret_cast<f16x4*>(dst + ((qg * QPW + i) * 64 + lane) * 16) = h;
+    }
+  };
+  // O^T += Dv(t) P^T(t).
+  auto multiply = [&](int t) {
+    const char* pb = lds + OFF_P + (t & 1) * PBYTES + lane * 16;
+#pragma unroll
+    for (int w = 0; w < KW; ++w)
+#pragma unroll
+      for (int i = 0; i < QB; ++i) {
+        const f16x8 pf = lds_v8<_Float16>(pb + (w * QB + i) * 1024);
+#pragma unroll
+        for (int f = 0; f < FB; ++f) acc[f][i] = Elem<_Float16>::mma(vreg[w][f], pf, acc[f][i]);
+      }
+    constexpr int FR = KW * QB, AHEAD = FR < 3 ? FR : 3;
+    __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+    for (int n = 0; n < FR - AHEAD; ++n) {
+      __builtin_amdgcn_sched_group_barrier(0x008, FB, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, AHEAD * FB, 0);
+  };
+
+  lds_barrier();   // key tiles 0 and 1
+  load_values(0);
+  __builtin_amdgcn_sched_barrier(0);
+  weights(0);
+
+  // Step t finds P(t) and the keys of t + 1 in LDS; the key buffer of t and
+  // the P buffer of t - 1 are free.
+  for (int t = 0; t + 1 < n_tiles; ++t) {
+    lds_barrier();
+    if (t + 2 < n_tiles) load_keys(t + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(t);
+    wait_vmem();
+    load_values(t + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    weights(t + 1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  lds_barrier();
+  multiply(n_tiles - 1);
+
+  // Row sums over the waves along the atoms (the first P buffer), then row
+  // norms over the waves along the coordinates (the second): r = O / l,
+  // z = r / max(||r||, eps).  Lane (c, g) holds coordinates
+  // 16 (wave FB + f) + 4g + e of row 16 i + c.
+  float* xl = reinterpret_cast<float*>(lds + OFF_P);
+  float* xn = reinterpret_cast<float*>(lds + OFF_P + PBYTES);
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < QPW; ++i) {
+    const float l = group_sum(l_part[i]);
+    if (g == 0) xl[kg * QT + (qg * QPW + i) * 16 + c] = l;
+  }
+  lds_barrier();
+  float w[QB];
+#pragma unroll
+  for (int i = 0; i < QB; ++i) {
+    float l = 0.f;
+#pragma unroll
+    for (int k = 0; k < NKG; ++k) l += xl[k * QT + i * 16 + c];
+    w[i] = 1.f / l;
+  }
+  if (p.flags & kRouteNormalizeOutput) {
+#pragma unroll
+    for (int i = 0; i < QB; ++i) {
+      float rs = 0.f;
+#pragma unroll
+      for (int f = 0; f < FB; ++f)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = acc[f][i][e] * w[i];
+          rs += v * v;
+        }
+      rs = group_sum(rs);
+      if (g == 0) xn[wave * QT + i * 16 + c] = rs;
+    }
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < QB; ++i) {
+      float rs = 0.f;
+#pragma unroll
+      for (int k = 0; k < kWaves; ++k) rs += xn[k * QT + i * 16 + c];
+      w[i] /= fmaxf(sqrtf(rs), p.eps);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < QB; ++i) {
+    const int64_t row = row0 + i * 16 + c;
+    if (row >= p.rows) continue;
+    TO* dst = static_cast<TO*>(p.out) + row * p.out_stride + wave * FB * 16 + 4 * g;
+#pragma unroll
+    for (int f = 0; f < FB; ++f) {
+      typename Elem<TO>::v4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = static_cast<TO>(acc[f][i][e] * w[i]);
+      *reinterpret_cast<typename Elem<TO>::v4*>(dst + f * 16) = o;
+    }
+  }
+}
+
+namespace {
+
+template <typename TX, typename TK, typename TO, int R, int QT, int KT, int QPW>
+void launch_k(const RouteArgs& a, hipStream_t s) {
+  static_assert(kAtomPad % KT == 0, "the bank is padded to whole tiles");
+  RouteTileParams p{};
+  p.x = a.x;
+  p.rows = a.rows;
+  p.x_stride = a.x_stride;
+  p.key_t = a.key_t;
+  p.value = static_cast<const _Float16*>(a.value);
+  p.M = a.M;
+  p.n_tiles = static_cast<int>((a.M + KT - 1) / KT);
+  p.beta_ptr = a.beta_ptr;
+  p.beta_dtype = a.beta_dtype;
+  p.beta_value = a.beta_value;
+  p.eps = a.eps;
+  p.flags = a.flags;
+  p.out = a.out;
+  p.out_stride = a.out_stride;
+  hipLaunchKernelGGL((route_tile_kernel<TX, TK, TO, R, QT, KT, QPW>), dim3(static_cast<unsigned>((a.rows + QT - 1) / QT)),
+                     dim3(kWaves * 64), 0, s, p);
+}
+
+// 512-wide rows: 64 rows per workgroup halve the reads of the dictionary, 32
+// spread fewer rows over twice the CUs (1536 atoms: 8192 rows 45 us in one
+// round of 32-row workgroups; in two rounds, 12000 rows take 83).
+constexpr int64_t kTileCUs = 256;
+
+template <typename TX, typename TK, typename TO>
+void launch_t(const RouteArgs& a, hipStream_t s) {
+  if (a.R == 256) {
+    launch_k<TX, TK, TO, 256, 32, 64, 1>(a, s);
+  } else if ((a.rows + 31) / 32 > kTileCUs) {
+    launch_k<TX, TK, TO, 512, 64, 32, 1>(a, s);
+  } else {
+    launch_k<TX, TK, TO, 512, 32, 64, 1>(a, s);
+  }
+}
+
+}  // namespace
+
+void launch_route_tile(const RouteArgs& a, hipStream_t s) {
+  if (a.x_dtype == kBF16) {
+    if (a.key_dtype == kF16) {
+      if (a.out_dtype == kF16) launch_t<__bf16, _Float16, _Float16>(a, s);
+      else launch_t<__bf16, _Float16, __bf16>(a, s);
+    } else {
+      if (a.out_dtype == kF16) launch_t<__bf16, __bf16, _Float16>(a, s);
+      else launch_t<__bf16, __bf16, __bf16>(a, s);
+    }
+  } else {
+    launch_t<_Float16, _Float16, _Float16>(a, s);
+  }
+}
+
+}  // namespace da
