@@ -478,7 +478,9 @@ __global__ __launch_bounds__(256) void attention_tile_merge_kernel(TileParams p)
     for (int k = 0; k < AHEAD; ++k)
 #pragma unroll
       for (int r = 0; r < RW; ++r) {
-        if (y + k >= n || !(l[k][r] > 0.f)) continue;   // a piece with every key of the row masked
+        // A piece with every key of the row masked has the sum 0; a NaN sum is
+        // a NaN score and goes on to the output, as it does without a split.
+        if (y + k >= n || l[k][r] == 0.f) continue;
         const float Mn = fmaxf(M[r], m[k][r]);
         const float f_old = M[r] == -INFINITY ? 0.f : exp2f(M[r] - Mn);
         const float wl = exp2f(m[k][r] - Mn) * l[k][r];
@@ -500,7 +502,7 @@ __global__ __launch_bounds__(256) void attention_tile_merge_kernel(TileParams p)
   for (int r = 0; r < RW; ++r) {
     const int tq = qt * QT + r0 + r * RPP;
     if (tq >= p.T) continue;
-    const float w = den[r] > 0.f ? 1.f / den[r] : 0.f;
+    const float w = den[r] == 0.f ? 0.f : 1.f / den[r];
     char* dst = static_cast<char*>(p.out) +
                 (b * p.out_stride_b + static_cast<int64_t>(tq) * p.out_stride_t + ds0 + d8) * ES;
     if constexpr (ES == 4) {

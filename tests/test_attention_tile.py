@@ -19,10 +19,12 @@ pytestmark = pytest.mark.gpu
 F16, BF16 = _lib.DA_F16, _lib.DA_BF16
 
 
-def _case(batch, maps, length, score_dim, value_dim, dtype, causal, log_scale, bound, out_f32=False):
+def _case(batch, maps, length, score_dim, value_dim, dtype, causal, log_scale, bound, out_f32=False, spoil=None):
     g = torch.Generator().manual_seed(length + score_dim)
     rows = torch.nn.functional.normalize(torch.randn(batch, length, 2, maps, score_dim, generator=g), dim=-1).half()
     value = torch.randn(batch, length, value_dim, generator=g).to(dtype)
+    if spoil is not None:
+        spoil(rows, value)
     scales = torch.linspace(log_scale - 0.4, log_scale + 0.4, maps) if maps > 1 else torch.tensor([log_scale])
     logits = torch.linspace(-0.7, 0.9, maps)
     padded = (length + 63) // 64 * 64
@@ -89,3 +91,32 @@ def test_attention_tile(case) -> None:
     # Without scratch the general kernel takes the call.
     general = call(0)
     assert np.linalg.norm(general - got) / np.linalg.norm(expected) <= 2 * bar
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])   # the fixed reference, and row maxima
+@pytest.mark.parametrize(("width", "causal"), [(256, True), (512, True), (256, False)])
+def test_attention_tile_nan_scores(dtype, width, causal) -> None:
+    """A NaN key reaches every query that sees it, a NaN query its own row, in
+    split and whole query tiles alike; no other row changes."""
+
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    print(f"[attention tile nan] {dtype} {width} causal {causal}", flush=True)
+    length, key_at, query_at = 2177, 1400, (5, 700, 1300)
+
+    def spoil(rows, value):
+        rows[0, key_at, 1] = float("nan")
+        for t in query_at:
+            rows[0, t, 0] = float("nan")
+
+    args = (1, 1, length, width, 512, dtype, causal, 2.77, 1.01)
+    call, need, _ = _case(*args)
+    clean = call(need)[0]
+    call, need, _ = _case(*args, spoil=spoil)
+    assert need > 0
+    got = call(need)[0]
+    bad = np.zeros(length, bool)
+    bad[key_at if causal else 0:] = True
+    bad[list(query_at)] = True
+    assert np.isnan(got[bad]).all(), np.flatnonzero(bad & ~np.isnan(got).all(axis=1))[:8]
+    np.testing.assert_array_equal(got[~bad], clean[~bad])
