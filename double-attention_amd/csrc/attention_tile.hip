@@ -52,6 +52,7 @@ struct TileParams {
   int n_pieces;         // pieces of every query tile otherwise
   int piece_len;        // key tiles per piece
   char* part;           // split: [sequence x slice][item] slots
+  int piece_es;         // bytes of a piece's element (2: the value type, 4: fp32)
   const void* scales;
   int scales_dtype;
   float scale_mult;
@@ -92,10 +93,23 @@ __host__ __device__ inline int64_t piece_slot_bytes(int QT, int DS, int es) {
   return static_cast<int64_t>(QT) * DS * es + 8 * static_cast<int64_t>(QT);
 }
 
+// Four features in fp32 or in the value type.
+template <typename TV>
+__device__ __forceinline__ void store_features(char* dst, int es, f32x4 v) {
+  if (es == 4) {
+    *reinterpret_cast<f32x4*>(dst) = v;
+  } else {
+    typename Elem<TV>::v4 h;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) h[r] = static_cast<TV>(v[r]);
+    *reinterpret_cast<typename Elem<TV>::v4*>(dst) = h;
+  }
+}
+
 }  // namespace
 
-// W: score width.  ES: bytes of an output element (2: TV, 4: fp32).
-template <typename TV, int W, int DS, int ES>
+// W: score width.
+template <typename TV, int W, int DS>
 __global__ __launch_bounds__(kTileWaves * 64) void attention_tile_kernel(TileParams p) {
   typedef _Float16 TQ;
   typedef typename Elem<TQ>::v8 q8;
@@ -390,9 +404,9 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_tile_kernel(TilePar
   char* slot = nullptr;
   if (partial) {
     slot = p.part + (static_cast<int64_t>(b * p.n_slices + slice) * p.items +
-                     tile_slot(it.qt, it.piece, p.piece_group, p.n_pieces)) * piece_slot_bytes(QT, DS, ES);
+                     tile_slot(it.qt, it.piece, p.piece_group, p.n_pieces)) * piece_slot_bytes(QT, DS, p.piece_es);
     if (kg == 0 && g == 0) {
-      float* stats = reinterpret_cast<float*>(slot + static_cast<int64_t>(QT) * DS * ES);
+      float* stats = reinterpret_cast<float*>(slot + static_cast<int64_t>(QT) * DS * p.piece_es);
 #pragma unroll
       for (int i = 0; i < QPW; ++i) {
         const int ql = (qg * QPW + i) * 16 + c;
@@ -404,6 +418,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_tile_kernel(TilePar
       }
     }
   }
+  const int es = partial ? p.piece_es : (p.flags & kAttnOutF32) ? 4 : 2;
 #pragma unroll
   for (int i = 0; i < QB; ++i) {
     float l = 0.f;
@@ -413,26 +428,16 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_tile_kernel(TilePar
     const int tq = q0 + i * 16 + c;
     const int64_t at = partial ? static_cast<int64_t>(i * 16 + c) * DS + wave * FB * 16
                                : b * p.out_stride_b + static_cast<int64_t>(tq) * p.out_stride_t + ds0 + wave * FB * 16;
-    char* dst = (partial ? slot : static_cast<char*>(p.out)) + at * ES;
+    char* dst = (partial ? slot : static_cast<char*>(p.out)) + at * es;
     if (!partial && tq >= p.T) continue;
 #pragma unroll
-    for (int f = 0; f < FB; ++f) {
-      const f32x4 o = acc[f][i] * w;
-      if constexpr (ES == 4) {
-        *reinterpret_cast<f32x4*>(dst + (f * 16 + 4 * g) * 4) = o;
-      } else {
-        typename Elem<TV>::v4 h;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) h[r] = static_cast<TV>(o[r]);
-        *reinterpret_cast<typename Elem<TV>::v4*>(dst + (f * 16 + 4 * g) * 2) = h;
-      }
-    }
+    for (int f = 0; f < FB; ++f) store_features<TV>(dst + (f * 16 + 4 * g) * es, es, acc[f][i] * w);
   }
 }
 
 // Merge of a query tile's pieces: O = sum 2^(m_c - M) l_c o_c / sum 2^(m_c - M) l_c
 // per row.
-template <typename TV, int DS, int ES>
+template <typename TV, int DS, int PE>
 __global__ __launch_bounds__(256) void attention_tile_merge_kernel(TileParams p) {
   // Eight features per lane; a wave takes 512 / DS rows at a time, RW times.
   constexpr int QT = kTileQueries, LPR = DS / 8, RPP = 64 / LPR, RW = 2, AHEAD = 2;
@@ -446,7 +451,7 @@ __global__ __launch_bounds__(256) void attention_tile_merge_kernel(TileParams p)
   const int lane = lane_id();
   const int d8 = (lane % LPR) * 8;
   const int r0 = (static_cast<int>(blockIdx.z) * 4 + uniform_wave()) * RW * RPP + lane / LPR;
-  const int64_t bytes = piece_slot_bytes(QT, DS, ES);
+  const int64_t bytes = piece_slot_bytes(QT, DS, PE);
   const char* base = p.part + (static_cast<int64_t>(blockIdx.x) * p.items + first) * bytes;
   float M[RW], den[RW], o[RW][8];
 #pragma unroll
@@ -460,18 +465,18 @@ __global__ __launch_bounds__(256) void attention_tile_merge_kernel(TileParams p)
     // The loads of AHEAD pieces fly together (past the last piece its own are
     // repeated and dropped).
     float m[AHEAD][RW], l[AHEAD][RW];
-    u32x4 v[AHEAD][RW][ES / 2];
+    u32x4 v[AHEAD][RW][PE / 2];
 #pragma unroll
     for (int k = 0; k < AHEAD; ++k) {
       const char* pc = base + min(y + k, n - 1) * bytes;
-      const float* stats = reinterpret_cast<const float*>(pc + static_cast<int64_t>(QT) * DS * ES);
+      const float* stats = reinterpret_cast<const float*>(pc + static_cast<int64_t>(QT) * DS * PE);
 #pragma unroll
       for (int r = 0; r < RW; ++r) {
         const int row = r0 + r * RPP;
         m[k][r] = stats[row];
         l[k][r] = stats[QT + row];
 #pragma unroll
-        for (int h = 0; h < ES / 2; ++h) v[k][r][h] = load16B(pc + (static_cast<int64_t>(row) * DS + d8) * ES + 16 * h);
+        for (int h = 0; h < PE / 2; ++h) v[k][r][h] = load16B(pc + (static_cast<int64_t>(row) * DS + d8) * PE + 16 * h);
       }
     }
 #pragma unroll
@@ -488,7 +493,7 @@ __global__ __launch_bounds__(256) void attention_tile_merge_kernel(TileParams p)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           float x;
-          if constexpr (ES == 4) {
+          if constexpr (PE == 4) {
             x = __uint_as_float(v[k][r][e >> 2][e & 3]);
           } else {
             x = static_cast<float>(__builtin_bit_cast(typename Elem<TV>::v8, v[k][r][0])[e]);
@@ -503,9 +508,10 @@ __global__ __launch_bounds__(256) void attention_tile_merge_kernel(TileParams p)
     const int tq = qt * QT + r0 + r * RPP;
     if (tq >= p.T) continue;
     const float w = den[r] == 0.f ? 0.f : 1.f / den[r];
+    const int es = (p.flags & kAttnOutF32) ? 4 : 2;
     char* dst = static_cast<char*>(p.out) +
-                (b * p.out_stride_b + static_cast<int64_t>(tq) * p.out_stride_t + ds0 + d8) * ES;
-    if constexpr (ES == 4) {
+                (b * p.out_stride_b + static_cast<int64_t>(tq) * p.out_stride_t + ds0 + d8) * es;
+    if (es == 4) {
       *reinterpret_cast<f32x4*>(dst) = f32x4{o[r][0], o[r][1], o[r][2], o[r][3]} * w;
       *reinterpret_cast<f32x4*>(dst + 16) = f32x4{o[r][4], o[r][5], o[r][6], o[r][7]} * w;
     } else {
@@ -524,11 +530,11 @@ constexpr int64_t kTileCUs = 256;
 // What a launch needs: value slice width and the split of its work.
 struct TilePlan {
   bool fits;
-  int ds, piece_group, n_pieces, piece_len, items;
+  int ds, piece_group, n_pieces, piece_len, items, piece_es;
   int64_t part_bytes;
 };
 
-TilePlan plan_tile(int64_t B, int64_t S, int64_t T, int64_t D, int64_t W, bool causal, int es) {
+TilePlan plan_tile(int64_t B, int64_t S, int64_t T, int64_t D, int64_t W, bool causal, int out_es) {
   TilePlan t{};
   // Sequences long enough to give every piece a run of key tiles.  Against
   // the general kernel (us, causal, bf16, D 512): 256-wide scores 1 x 2048
@@ -567,26 +573,32 @@ TilePlan plan_tile(int64_t B, int64_t S, int64_t T, int64_t D, int64_t W, bool c
     t.n_pieces = static_cast<int>((n_last + t.piece_len - 1) / t.piece_len);
     t.items = static_cast<int>(n_qt * t.n_pieces);
   }
-  if (t.items > n_qt) t.part_bytes = B * slices * t.items * piece_slot_bytes(kTileQueries, t.ds, es);
+  // Pieces are fp32, unless the general kernel would split this call's keys
+  // too and round its pieces to the output's 16 bits.  Their error against 64
+  // bits is then the same (bf16, causal: 1 x 8192 tokens 2.35e-3 there, 2.38e-3
+  // here; 4 x 2048 2.40e-3 both); where it does not split, 16-bit pieces would add
+  // a rounding (2 x 2500 without a mask 2.36e-3 there, 2.89e-3 with them).
+  t.piece_es = out_es == 2 && plan_attention(B, S, T, D, W, false, causal, true, 2).part_bytes > 0 ? 2 : 4;
+  if (t.items > n_qt) t.part_bytes = B * slices * t.items * piece_slot_bytes(kTileQueries, t.ds, t.piece_es);
   return t;
 }
 
-template <typename TV, int W, int DS, int ES>
+template <typename TV, int W, int DS>
 void launch_tile_k(const AttentionArgs& a, const TilePlan& t, const TileParams& p, hipStream_t s) {
-  hipLaunchKernelGGL((attention_tile_kernel<TV, W, DS, ES>), dim3(static_cast<unsigned>(a.B * p.n_slices * p.items)),
+  hipLaunchKernelGGL((attention_tile_kernel<TV, W, DS>), dim3(static_cast<unsigned>(a.B * p.n_slices * p.items)),
                      dim3(kTileWaves * 64), 0, s, p);
-  if (t.part_bytes > 0)
-    hipLaunchKernelGGL((attention_tile_merge_kernel<TV, DS, ES>),
-                       dim3(static_cast<unsigned>(a.B * p.n_slices), static_cast<unsigned>(p.n_qt),
-                            static_cast<unsigned>(kTileQueries / (8 * (512 / DS)))),
-                       dim3(256), 0, s, p);
+  if (t.part_bytes == 0) return;
+  const dim3 merge(static_cast<unsigned>(a.B * p.n_slices), static_cast<unsigned>(p.n_qt),
+                   static_cast<unsigned>(kTileQueries / (8 * (512 / DS))));
+  if (t.piece_es == 4) hipLaunchKernelGGL((attention_tile_merge_kernel<TV, DS, 4>), merge, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((attention_tile_merge_kernel<TV, DS, 2>), merge, dim3(256), 0, s, p);
 }
 
-template <typename TV, int ES>
+template <typename TV>
 void launch_tile_t(const AttentionArgs& a, const TilePlan& t, const TileParams& p, hipStream_t s) {
-  if (a.RP == 512) launch_tile_k<TV, 512, 256, ES>(a, t, p, s);
-  else if (t.ds == 512) launch_tile_k<TV, 256, 512, ES>(a, t, p, s);
-  else launch_tile_k<TV, 256, 256, ES>(a, t, p, s);
+  if (a.RP == 512) launch_tile_k<TV, 512, 256>(a, t, p, s);
+  else if (t.ds == 512) launch_tile_k<TV, 256, 512>(a, t, p, s);
+  else launch_tile_k<TV, 256, 256>(a, t, p, s);
 }
 
 }  // namespace
@@ -617,6 +629,7 @@ bool launch_attention_tile(const AttentionArgs& a, void* workspace, int64_t work
   p.piece_group = t.piece_group;
   p.n_pieces = t.n_pieces;
   p.piece_len = t.piece_len;
+  p.piece_es = t.piece_es;
   p.part = static_cast<char*>(workspace);
   p.scales = a.scales;
   p.scales_dtype = a.scales_dtype;
@@ -626,13 +639,8 @@ bool launch_attention_tile(const AttentionArgs& a, void* workspace, int64_t work
   p.out = a.out;
   p.out_stride_b = a.out_stride_b;
   p.out_stride_t = a.out_stride_t;
-  if (a.v_dtype == kBF16) {
-    if (es == 4) launch_tile_t<__bf16, 4>(a, t, p, stream);
-    else launch_tile_t<__bf16, 2>(a, t, p, stream);
-  } else {
-    if (es == 4) launch_tile_t<_Float16, 4>(a, t, p, stream);
-    else launch_tile_t<_Float16, 2>(a, t, p, stream);
-  }
+  if (a.v_dtype == kBF16) launch_tile_t<__bf16>(a, t, p, stream);
+  else launch_tile_t<_Float16>(a, t, p, stream);
   return true;
 }
 

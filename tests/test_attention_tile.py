@@ -120,3 +120,26 @@ def test_attention_tile_nan_scores(dtype, width, causal) -> None:
     bad[list(query_at)] = True
     assert np.isnan(got[bad]).all(), np.flatnonzero(bad & ~np.isnan(got).all(axis=1))[:8]
     np.testing.assert_array_equal(got[~bad], clean[~bad])
+
+
+@pytest.mark.parametrize("case", [
+    # batch, length, score width, value width, causal: the general kernel splits none of these
+    (2, 2500, 256, 512, False),
+    (3, 2500, 256, 512, True),
+    (4, 2048, 512, 512, False),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_attention_tile_pieces_are_fp32(case, dtype) -> None:
+    """Where only this kernel splits the keys, a 16-bit output is its fp32 one
+    rounded once: the pieces hold fp32."""
+
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    batch, length, width, value_dim, causal = case
+    print(f"[attention tile pieces] {case} {dtype}", flush=True)
+    args = (batch, 1, length, width, value_dim, dtype, causal, 2.77, 1.01)
+    call, need, _ = _case(*args)
+    exact, need32, _ = _case(*args, out_f32=True)
+    assert need > 0 and need32 > 0   # both split
+    rounded = torch.from_numpy(exact(need32)).to(dtype).float().numpy()
+    np.testing.assert_array_equal(call(need), rounded)
