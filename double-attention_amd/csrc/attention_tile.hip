@@ -518,7 +518,10 @@ __global__ __launch_bounds__(256) void attention_tile_merge_kernel(TileParams p)
       typename Elem<TV>::v8 h;
 #pragma unroll
       for (int e = 0; e < 8; ++e) h[e] = static_cast<TV>(o[r][e] * w);
-      *reinterpret_cast<typename Elem<TV>::v8*>(dst) = h;
+      // 16-bit outputs and their strides may be 8-byte aligned only.
+      const u32x4 bits = __builtin_bit_cast(u32x4, h);
+      *reinterpret_cast<u32x2*>(dst) = u32x2{bits[0], bits[1]};
+      *reinterpret_cast<u32x2*>(dst + 8) = u32x2{bits[2], bits[3]};
     }
   }
 }

@@ -19,7 +19,8 @@ pytestmark = pytest.mark.gpu
 F16, BF16 = _lib.DA_F16, _lib.DA_BF16
 
 
-def _case(batch, maps, length, score_dim, value_dim, dtype, causal, log_scale, bound, out_f32=False, spoil=None):
+def _case(batch, maps, length, score_dim, value_dim, dtype, causal, log_scale, bound, out_f32=False, spoil=None,
+          pad=0):
     g = torch.Generator().manual_seed(length + score_dim)
     rows = torch.nn.functional.normalize(torch.randn(batch, length, 2, maps, score_dim, generator=g), dim=-1).half()
     value = torch.randn(batch, length, value_dim, generator=g).to(dtype)
@@ -36,7 +37,10 @@ def _case(batch, maps, length, score_dim, value_dim, dtype, causal, log_scale, b
     d = torch.device("cuda:0")
     rd, td, sd, ld = rows.to(d), tiles.to(d), scales.to(d), logits.to(d)
     out_dtype = torch.float32 if out_f32 else dtype
-    out = torch.full((batch, length, value_dim), float("nan"), dtype=out_dtype, device=d)
+    # `pad` features before the output's first and after each row's last.
+    whole = torch.full((pad + batch * length * (value_dim + pad),), float("nan"), dtype=out_dtype, device=d)
+    framed = whole[pad:].view(batch, length, value_dim + pad)
+    out = framed[..., :value_dim]
     flags = _lib.DA_ATTN_SCALES_ARE_LOG | (_lib.DA_ATTN_CAUSAL if causal else 0)
     flags |= (_lib.DA_ATTN_MIX if maps > 1 else 0) | (_lib.DA_ATTN_OUT_F32 if out_f32 else 0)
     lib = _lib.get()
@@ -45,7 +49,7 @@ def _case(batch, maps, length, score_dim, value_dim, dtype, causal, log_scale, b
     width = maps * score_dim
 
     def call(nbytes):
-        out.fill_(float("nan"))
+        whole.fill_(float("nan"))
         _lib.check(
             lib.da_routed_attention(
                 rd.data_ptr(), rd.data_ptr() + width * 2, length * 2 * width, 2 * width, score_dim, 1, score_dim,
@@ -57,6 +61,7 @@ def _case(batch, maps, length, score_dim, value_dim, dtype, causal, log_scale, b
             "attention",
         )
         torch.cuda.synchronize()
+        assert whole[:pad].isnan().all() and framed[..., value_dim:].isnan().all()
         return out.float().cpu().numpy()
 
     q, k = (rows[:, :, i].permute(0, 2, 1, 3).float().numpy() for i in (0, 1))
@@ -143,3 +148,17 @@ def test_attention_tile_pieces_are_fp32(case, dtype) -> None:
     assert need > 0 and need32 > 0   # both split
     rounded = torch.from_numpy(exact(need32)).to(dtype).float().numpy()
     np.testing.assert_array_equal(call(need), rounded)
+
+
+@pytest.mark.parametrize("batch", [1, 24])   # split keys (the merge stores the output), whole ones
+def test_attention_tile_eight_byte_outputs(batch) -> None:
+    """16-bit outputs that start and step at multiples of 8 bytes, not of 16."""
+
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    print(f"[attention tile 8-byte outputs] batch {batch}", flush=True)
+    args = (batch, 1, 1055, 512, 256, torch.bfloat16, False, 3.1, 1.01)
+    plain, need, _ = _case(*args)
+    assert (need > 0) == (batch == 1)
+    framed, _, _ = _case(*args, pad=4)
+    np.testing.assert_array_equal(framed(need), plain(need))
