@@ -136,7 +136,6 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_tile_kernel(TilePar
   const int lane = lane_id();
   const int c = lane & 15, g = lane >> 4;
   const int wave = uniform_wave();
-  const int tid = static_cast<int>(threadIdx.x);
   const int kg = wave % NKG, qg = wave / NKG;   // this wave's score blocks
   const ScalarHalves scale_raw = fetch_scalar(p.scales, p.scales_dtype, 0);   // issued first, used later
   const bool causal = p.flags & kAttnCausal;
@@ -206,7 +205,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_tile_kernel(TilePar
     for (int kk = 0; kk < KS; ++kk) qf[i][kk] = load8(src + kk * 32);
   }
   load_keys(kt0);
-  load_keys(min(kt0 + 1, kt1 - 1));
+  if (kt0 + 1 < kt1) load_keys(kt0 + 1);
   // Nothing that uses a loaded value moves above the loads' issue.
   __builtin_amdgcn_sched_barrier(0);
   wait_vmem();
@@ -278,7 +277,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_tile_kernel(TilePar
     for (int kt = kt0; kt < kt1; ++kt) {
       wait_vmem();
       lds_barrier();
-      if (kt > kt0) load_keys(min(kt + 1, kt1 - 1));
+      if (kt > kt0 && kt + 1 < kt1) load_keys(kt + 1);
       f32x4 st[QPW][KPW];
       scores(kt, st);
 #pragma unroll
@@ -308,7 +307,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_tile_kernel(TilePar
     // of both key buffers; the barrier below is past the exchange's).
     wait_vmem();
     load_keys(kt0);
-    load_keys(min(kt0 + 1, kt1 - 1));
+    if (kt0 + 1 < kt1) load_keys(kt0 + 1);
     wait_vmem();
   }
 
@@ -372,13 +371,12 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_tile_kernel(TilePar
   probabilities(kt0);
 
   // Step kt finds P(kt) and the keys of kt + 1 in LDS; the key buffer of kt
-  // and the P buffer of kt - 1 are free.  The key loads land behind the
-  // step's products; the value loads of kt + 1 follow them.  The two waves of
-  // a SIMD (w and w + 4) take the halves of a step in opposite order, so one's
-  // exponentials run beside the other's MFMAs.
+  // and the P buffer of kt - 1 are free.  The key loads (none past the last
+  // tile: its buffer is still being read) land behind the step's products; the
+  // value loads of kt + 1 follow them.
   for (int kt = kt0; kt + 1 < kt1; ++kt) {
     lds_barrier();
-    load_keys(min(kt + 2, kt1 - 1));
+    if (kt + 2 < kt1) load_keys(kt + 2);
     __builtin_amdgcn_sched_barrier(0);
     multiply(kt);
     wait_vmem();
