@@ -927,7 +927,7 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnParams p) {
       }
 #pragma unroll
       for (int r = 0; r < RW; ++r) {
-        if (m[r] == -INFINITY) continue;   // a piece with every key masked
+        if (l[r] == 0.f) continue;   // a piece with every key masked (a NaN query has no maximum either, but a NaN sum)
         const float Mn = fmaxf(M[r], m[r]);
         const float f_old = M[r] == -INFINITY ? 0.f : exp2f(M[r] - Mn);
         const float wl = exp2f(m[r] - Mn) * l[r];
@@ -940,7 +940,7 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnParams p) {
     const float wmap = MULTI ? map_weight(p, s) : 1.f;
 #pragma unroll
     for (int r = 0; r < RW; ++r) {
-      const float w = wmap * (den[r] > 0.f ? 1.f / den[r] : 0.f);
+      const float w = wmap * (den[r] == 0.f ? 0.f : 1.f / den[r]);
 #pragma unroll
       for (int k = 0; k < NV; ++k) out[r][k] += o[r][k] * w;
     }

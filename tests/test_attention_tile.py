@@ -99,15 +99,21 @@ def test_attention_tile(case) -> None:
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])   # the fixed reference, and row maxima
-@pytest.mark.parametrize(("width", "causal"), [(256, True), (512, True), (256, False)])
-def test_attention_tile_nan_scores(dtype, width, causal) -> None:
+@pytest.mark.parametrize(("length", "width", "causal"), [
+    (2177, 256, True),
+    (2177, 512, True),
+    (2177, 256, False),
+    (1500, 256, True),    # the general kernel
+    (1500, 256, False),
+])
+def test_split_attention_nan_scores(dtype, length, width, causal) -> None:
     """A NaN key reaches every query that sees it, a NaN query its own row, in
     split and whole query tiles alike; no other row changes."""
 
     if not torch.cuda.is_available():
         pytest.skip("needs a GPU")
-    print(f"[attention tile nan] {dtype} {width} causal {causal}", flush=True)
-    length, key_at, query_at = 2177, 1400, (5, 700, 1300)
+    print(f"[split attention nan] {dtype} {length} {width} causal {causal}", flush=True)
+    key_at, query_at = 1400, (5, 700, 1300)
 
     def spoil(rows, value):
         rows[0, key_at, 1] = float("nan")
