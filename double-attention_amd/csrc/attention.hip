@@ -1393,6 +1393,68 @@ AttnPlan plan_attention(int64_t B, int64_t S, int64_t T, int64_t D, int64_t RP, 
   return plan;
 }
 
+double dealt_steps(int64_t B, int64_t slices, int64_t tiles, int64_t slots, double longest, double fall) {
+  const int64_t per = tiles * slices, all = B * per;
+  auto cost = [&](int64_t i) { return longest - fall * static_cast<double>(i % per / slices); };
+  // Steps of the workgroups before i.
+  auto before = [&](int64_t i) {
+    const double n = static_cast<double>(tiles), y = static_cast<double>(i % per / slices);
+    return static_cast<double>(i / per * slices) * (n * longest - fall * n * (n - 1) / 2) +
+           static_cast<double>(slices) * (y * longest - fall * y * (y - 1) / 2) +
+           static_cast<double>(i % slices) * cost(i);
+  };
+  double most = 0;
+  for (int64_t x = 0; x < kXcds; ++x) {
+    const int64_t a = x * (all / kXcds) + std::min(x, all % kXcds), n = all / kXcds + (x < all % kXcds), b = a + n;
+    if (n == 0) break;
+    const int64_t next = (a / per + 1) * per;   // the next sequence's first (longest) workgroup
+    double steps;
+    if (fall == 0) {
+      steps = static_cast<double>((n + slots - 1) / slots) * longest;
+    } else if (n <= slots) {
+      steps = std::max(cost(a), next < b ? cost(next) : 0);
+    } else {
+      // The largest of: an even share of the steps; the first workgroup past
+      // the slots, which starts as the shortest of those running ends; the
+      // rounds of a stretch of one sequence; the last sequence's longest one.
+      const double shortest = next <= a + slots ? std::min(cost(next - 1), cost(a + slots - 1)) : cost(a + slots - 1);
+      steps = std::max({(before(b) - before(a)) / static_cast<double>(slots), cost(a), shortest + cost(a + slots)});
+      if (next >= b)
+        steps = std::max(steps, static_cast<double>((n + slots - 1) / slots) * cost(b - 1) + 0.75 * (cost(a) - cost(b - 1)));
+      const int64_t last = (b - 1) / per * per;
+      if (last > a + slots) steps = std::max(steps, (before(last) - before(a)) / static_cast<double>(slots) + cost(last));
+    }
+    most = std::max(most, steps);
+  }
+  return most;
+}
+
+// Times fitted to 1160 shapes (T 1024 to 8192, D 256 to 1024, 1 to 32 sequences,
+// with and without a mask), most of them within 3 %.
+double attention_general_us(int64_t B, int64_t T, int64_t D, int64_t RP, bool causal, int piece_bytes,
+                            AttnExponents mode) {
+  const AttnPlan p = plan_attention(B, 1, T, D, RP, false, causal, true, piece_bytes);
+  // us per step (one key tile of a workgroup), by exponents: 512-wide scores,
+  // the plain grid, two sub-streams, the stream split of two slice widths.
+  const int m = static_cast<int>(mode);
+  constexpr double kWide[3] = {1.20, 1.55, 1.33}, kPlain[3] = {1.00, 1.42, 1.42}, kSub[3] = {0.88, 1.06, 1.06},
+                   kStream128[3] = {0.78, 1.00, 1.00}, kStream256[3] = {0.96, 1.42, 1.42};
+  const int64_t slices = D / p.ds, cus = kCUs / kXcds;
+  const int64_t qtile = p.nw * kAttnQW, n_last = host_key_tiles(p.n_qt - 1, qtile, T, causal);
+  if (p.stream_len > 0) {
+    // A run that ends inside a query tile loads the next one's queries.
+    const double start = causal ? 24 : n_last % p.stream_len ? 19 : 13;
+    const double step = RP == 512 ? kWide[m] : p.ds == 256 ? kStream256[m] : kStream128[m];
+    return start + 0.25e-6 * static_cast<double>(p.part_bytes) +
+           step * dealt_steps(B, slices, p.n_seg, cus, p.stream_len + kLaunchSteps, 0);
+  }
+  const double start = p.sub == 2 ? 5 : RP == 512 ? 6 : 9;
+  const double step = RP == 512 ? kWide[m] : p.sub == 2 ? kSub[m] : kPlain[m];
+  const double fall = causal ? static_cast<double>(qtile) / kKeyTile / p.sub : 0;
+  return start + step * dealt_steps(B, slices, p.n_qt, cus * (4 / (p.nw * p.sub)),
+                                    static_cast<double>((n_last + p.sub - 1) / p.sub) + kLaunchSteps, fall);
+}
+
 template <typename TQ, typename TV, int RP>
 static void launch_attn_short_d(const AttentionArgs& a, AttnParams& p, hipStream_t s) {
   if (a.D % 128 == 0) launch_attn_short<TQ, TV, RP, 128>(a, p, s);

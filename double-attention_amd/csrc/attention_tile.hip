@@ -537,11 +537,7 @@ struct TilePlan {
 
 TilePlan plan_tile(int64_t B, int64_t S, int64_t T, int64_t D, int64_t W, bool causal, int out_es) {
   TilePlan t{};
-  // Sequences long enough to give every piece a run of key tiles.  Against
-  // the general kernel (us, causal, bf16, D 512): 256-wide scores 1 x 2048
-  // tokens 37 / 43, 2 x 2500 42 / 54, 1 x 8192 75 / 91, but 4 x 1024 35 / 21;
-  // 512-wide scores (whose tiles fill a CU's LDS there) 2 x 1100 38 / 52, 4 x
-  // 2048 57 / 68.  Without a mask 8 x 2048 68 / 79.
+  // Sequences long enough to give every piece a run of key tiles.
   if (S != 1 || D % 256 || !(W == 256 || W == 512) || T < (W == 512 ? 1024 : 2048)) return t;
   t.fits = true;
   // Value slices as wide as the registers allow: the scores are formed once
@@ -569,19 +565,65 @@ TilePlan plan_tile(int64_t B, int64_t S, int64_t T, int64_t D, int64_t W, bool c
       t.items = static_cast<int>(items(group));
     }
   } else {
-    const int64_t pieces = (n_last + share - 1) / share;
-    t.piece_len = static_cast<int>((n_last + pieces - 1) / pieces);
-    t.n_pieces = static_cast<int>((n_last + t.piece_len - 1) / t.piece_len);
-    t.items = static_cast<int>(n_qt * t.n_pieces);
+    // The fewest pieces with the shortest rounds of CUs: a few workgroups past
+    // a round cost a whole one (bf16, 256-wide scores, 3 x 2500 tokens, D 256: five
+    // pieces, 300 workgroups, 57 us; four, 240 workgroups, 40 us).
+    double best = 0;
+    for (int64_t pieces = 1; pieces <= (n_last + share - 1) / share; ++pieces) {
+      const int64_t len = (n_last + pieces - 1) / pieces, n = (n_last + len - 1) / len;
+      const double steps = dealt_steps(B, slices, n_qt * n, kTileCUs / kXcds, static_cast<double>(len) + kLaunchSteps, 0);
+      if (pieces > 1 && steps >= best) continue;
+      best = steps;
+      t.piece_len = static_cast<int>(len);
+      t.n_pieces = static_cast<int>(n);
+      t.items = static_cast<int>(n_qt * n);
+    }
   }
+  if (t.items == n_qt) return t;
   // Pieces are fp32, unless the general kernel would split this call's keys
   // too and round its pieces to the output's 16 bits.  Their error against 64
   // bits is then the same (bf16, causal: 1 x 8192 tokens 2.35e-3 there, 2.38e-3
   // here; 4 x 2048 2.40e-3 both); where it does not split, 16-bit pieces would add
   // a rounding (2 x 2500 without a mask 2.36e-3 there, 2.89e-3 with them).
   t.piece_es = out_es == 2 && plan_attention(B, S, T, D, W, false, causal, true, 2).part_bytes > 0 ? 2 : 4;
-  if (t.items > n_qt) t.part_bytes = B * slices * t.items * piece_slot_bytes(kTileQueries, t.ds, t.piece_es);
+  t.part_bytes = B * slices * t.items * piece_slot_bytes(kTileQueries, t.ds, t.piece_es);
   return t;
+}
+
+// As attention_general_us, fitted to the same shapes.
+double tile_us(const TilePlan& t, int64_t B, int64_t T, int64_t D, int64_t W, bool causal, bool fixed) {
+  const double step = W == 512 ? (fixed ? 1.47 : 2.26) : t.ds == 512 ? (fixed ? 1.26 : 1.85) : (fixed ? 1.03 : 1.53);
+  const int64_t n_qt = (T + kTileQueries - 1) / kTileQueries;
+  const double fall = causal && t.items == n_qt ? kTileQueries / kTileKeys : 0;
+  const double steps = dealt_steps(B, D / t.ds, t.items, kTileCUs / kXcds, t.piece_len + kLaunchSteps, fall);
+  if (t.part_bytes == 0) return (fixed ? 6 : 1) + step * steps;
+  const double start = W == 512 ? 8.5 : t.ds == 512 ? 13 : 10, per_mb = W == 512 ? 0.30 : t.ds == 512 ? 0.15 : 0.25;
+  return start + per_mb * 1e-6 * static_cast<double>(t.part_bytes) + step * steps;
+}
+
+// Whether this kernel beats the general one, by the predicted times of both.
+// It forms the scores fewer times, but the general kernel's smaller query tiles
+// fill the chip better in some calls, above all where its value slices are as
+// wide (us, bf16, here / there: 4 x 5000 causal, 256-wide scores, D 768 269 / 245;
+// 1 x 2048 without a mask, D 512 37.6 / 33.3; but 1 x 8192 causal 76 / 93).  With row
+// maxima (fp16 values, or no bound) it forms them twice, and the general one
+// rescales as it goes: fp16, 1 x 8192 causal 98 / 121 at 256-wide scores, 234 / 206 at
+// 512-wide.  A bf16 call with a bound runs fixed exponents up to a gamma of about
+// 41 and maxima past it, which only the device knows: it has to win with the
+// one and not lose 10 % with the other.  Over the shapes that the constants
+// were fitted to, the slowest choices are 6 % over the general kernel's time (a
+// few with fp16 values or no bound up to 12 %), where taking every call was up
+// to 62 %.
+bool tile_wins(const TilePlan& t, int64_t B, int64_t T, int64_t D, int64_t W, bool causal, int out_es, bool bf16,
+               bool bounded) {
+  auto ratio = [&](AttnExponents mode) {
+    return tile_us(t, B, T, D, W, causal, mode == AttnExponents::kFixed) /
+           attention_general_us(B, T, D, W, causal, out_es, mode);
+  };
+  if (!bf16) return ratio(AttnExponents::kMaximaF16) < 1;
+  if (!bounded) return ratio(AttnExponents::kMaximaBf16) < 1;
+  // The prediction for 512-wide scores is on the high side.
+  return ratio(AttnExponents::kFixed) < (W == 512 ? 1.05 : 1) && ratio(AttnExponents::kMaximaBf16) < 1.1;
 }
 
 template <typename TV, int W, int DS>
@@ -605,7 +647,11 @@ void launch_tile_t(const AttentionArgs& a, const TilePlan& t, const TileParams& 
 }  // namespace
 
 int64_t attention_tile_bytes(int64_t B, int64_t S, int64_t T, int64_t D, int64_t RP, bool causal, int es) {
-  return plan_tile(B, S, T, D, RP, causal, es).part_bytes;
+  const TilePlan t = plan_tile(B, S, T, D, RP, causal, es);
+  if (t.part_bytes == 0) return 0;
+  const bool taken = tile_wins(t, B, T, D, RP, causal, es, true, true) || tile_wins(t, B, T, D, RP, causal, es, true, false) ||
+                     tile_wins(t, B, T, D, RP, causal, es, false, false);
+  return taken ? t.part_bytes : 0;
 }
 
 bool launch_attention_tile(const AttentionArgs& a, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
@@ -614,6 +660,7 @@ bool launch_attention_tile(const AttentionArgs& a, void* workspace, int64_t work
   if (a.qk_dtype != kF16 || a.qk_stride_t * 2 * kTileKeys > INT32_MAX) return false;
   const TilePlan t = plan_tile(a.B, a.S, a.T, a.D, a.RP, a.flags & kAttnCausal, es);
   if (!t.fits || t.part_bytes > workspace_bytes) return false;
+  if (!tile_wins(t, a.B, a.T, a.D, a.RP, a.flags & kAttnCausal, es, a.v_dtype == kBF16, a.score_bound > 0.f)) return false;
   if (static_cast<int64_t>(a.B) * (a.D / t.ds) * t.items > INT32_MAX) return false;
   TileParams p{};
   p.q = a.q;

@@ -282,10 +282,20 @@ AttnPlan plan_attention(int64_t B, int64_t S, int64_t T, int64_t D, int64_t RP, 
 // `scratch`: device scratch of the call, or nullptr.  A kernel or split that
 // needs more than scratch_bytes is not taken.
 void launch_routed_attention(const AttentionArgs& a, void* scratch, int64_t scratch_bytes, hipStream_t stream);
+// Predicted times of one-map calls that either attention kernel takes, to
+// choose by.  Workgroups are dealt in order to eight XCDs of `slots` each;
+// a (sequence, slice) has `tiles` of them, of `longest` steps and `fall` fewer
+// each (a causal problem, heaviest first).  Steps until the last one is done:
+double dealt_steps(int64_t B, int64_t slices, int64_t tiles, int64_t slots, double longest, double fall);
+constexpr double kLaunchSteps = 4;   // a workgroup's start and end, in steps
+// Exponents against a fixed reference, or with row maxima (bf16, fp16 values).
+enum class AttnExponents { kFixed, kMaximaBf16, kMaximaF16 };
+double attention_general_us(int64_t B, int64_t T, int64_t D, int64_t RP, bool causal, int piece_bytes,
+                            AttnExponents mode);
 // The eight-wave kernel (attention_tile.hip): fp16 queries and keys, one map
 // over a long sequence.  Scratch bytes of a call with outputs of es bytes (0:
-// none, or not taken), and the launch itself: false when the call is not one
-// it takes, or needs more scratch than it is given.
+// none, or taken for no type of values), and the launch itself: false when the
+// call is not one it takes, or needs more scratch than it is given.
 int64_t attention_tile_bytes(int64_t B, int64_t S, int64_t T, int64_t D, int64_t RP, bool causal, int es);
 bool launch_attention_tile(const AttentionArgs& a, void* workspace, int64_t workspace_bytes, hipStream_t stream);
 

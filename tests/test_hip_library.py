@@ -119,6 +119,20 @@ def test_attention_rejects_bad_arguments_before_launch() -> None:
     assert h.da_routed_attention(*long_ctx) == -5
 
 
+def test_attention_scratch_follows_the_rule_between_kernels() -> None:
+    """The long-sequence kernel asks for scratch only where it is the faster
+    one in some type, and for pieces that fill whole rounds of the 256 CUs."""
+
+    h = lib.get()
+    # 4 x 2048 tokens, D 256, no mask: the general kernel's two sub-streams win,
+    # without scratch.
+    assert h.da_attention_workspace_bytes(4, 1, 2048, 256, 256, 0) == 0
+    # 3 x 2500 tokens, D 256, no mask: 20 query tiles x 3 sequences x 4 pieces of
+    # 128 x 256 floats and two floats per row (five pieces would take two rounds).
+    slot = 128 * 256 * 4 + 128 * 8
+    assert h.da_attention_workspace_bytes(3, 1, 2500, 256, 256, 0) == 3 * 20 * 4 * slot
+
+
 def test_forward_rejects_small_workspace() -> None:
     h = lib.get()
     f = _fake()
