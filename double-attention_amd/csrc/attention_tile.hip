@@ -170,9 +170,10 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_tile_kernel(TilePar
     KTile::slot_chunk((i * kTileWaves + wave) * 64 + lane, row, ck);
     koff[i] = static_cast<uint32_t>(row * kstride + ck * 16);
   }
-  // Keys of tile kt into its buffer (the parity of kt).
+  // Keys of tile kt into its buffer (the parity of kt).  Past the run's last
+  // tile that one is loaded again, into a buffer that nothing reads any more.
   auto load_keys = [&](int kt) {
-    const int k0 = kt * KT;
+    const int k0 = min(kt, kt1 - 1) * KT;
     const char* src = uniform_ptr(kbase + static_cast<int64_t>(k0) * kstride);
     char* dst = lds + (kt & 1) * KTile::BYTES + wave * 1024;
     if (k0 + KT <= p.T) {
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_tile_kernel(TilePar
     for (int kk = 0; kk < KS; ++kk) qf[i][kk] = load8(src + kk * 32);
   }
   load_keys(kt0);
-  if (kt0 + 1 < kt1) load_keys(kt0 + 1);
+  load_keys(kt0 + 1);
   // Nothing that uses a loaded value moves above the loads' issue.
   __builtin_amdgcn_sched_barrier(0);
   wait_vmem();
@@ -277,7 +278,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_tile_kernel(TilePar
     for (int kt = kt0; kt < kt1; ++kt) {
       wait_vmem();
       lds_barrier();
-      if (kt > kt0 && kt + 1 < kt1) load_keys(kt + 1);
+      if (kt > kt0) load_keys(kt + 1);
       f32x4 st[QPW][KPW];
       scores(kt, st);
 #pragma unroll
@@ -307,7 +308,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_tile_kernel(TilePar
     // of both key buffers; the barrier below is past the exchange's).
     wait_vmem();
     load_keys(kt0);
-    if (kt0 + 1 < kt1) load_keys(kt0 + 1);
+    load_keys(kt0 + 1);
     wait_vmem();
   }
 
@@ -371,12 +372,11 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_tile_kernel(TilePar
   probabilities(kt0);
 
   // Step kt finds P(kt) and the keys of kt + 1 in LDS; the key buffer of kt
-  // and the P buffer of kt - 1 are free.  The key loads (none past the last
-  // tile: its buffer is still being read) land behind the step's products; the
-  // value loads of kt + 1 follow them.
+  // and the P buffer of kt - 1 are free.  The key loads land behind the
+  // step's products; the value loads of kt + 1 follow them.
   for (int kt = kt0; kt + 1 < kt1; ++kt) {
     lds_barrier();
-    if (kt + 2 < kt1) load_keys(kt + 2);
+    load_keys(kt + 2);
     __builtin_amdgcn_sched_barrier(0);
     multiply(kt);
     wait_vmem();
