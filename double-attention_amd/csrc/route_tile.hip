@@ -54,9 +54,7 @@ struct RouteTileParams {
 
 }  // namespace
 
-// QPW: row blocks (of 16) of a wave's score blocks; every key fragment read
-// feeds QPW MFMAs.
-template <typename TX, typename TK, typename TO, int R, int QT, int KT, int QPW>
+template <typename TX, typename TK, typename TO, int R, int QT, int KT>
 __global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams p) {
   // x and out may alias (in-place routing): the workgroup has read its rows
   // into VGPRs, a barrier or more before any of its waves writes one.
@@ -64,7 +62,7 @@ __global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams
   constexpr int QB = QT / 16;                  // row blocks
   constexpr int KW = KT / 32;                  // 32-atom windows of a step
   constexpr int NKG = KT / 16;                 // waves along the atoms, one 16-atom block each
-  static_assert(NKG * (QB / QPW) == kWaves, "the score blocks go round the waves");
+  static_assert(NKG * QB == kWaves, "a score block per wave");
   constexpr int KS = R / 32;
   constexpr int FB = R / 128;                  // 16-coordinate blocks per wave
   typedef XorTile<KT, R / 8, true> KTile;
@@ -78,21 +76,20 @@ __global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams
   const int lane = lane_id();
   const int c = lane & 15, g = lane >> 4;
   const int wave = uniform_wave();
-  const int kg = wave % NKG, qg = wave / NKG;   // this wave's score blocks
+  const int kg = wave % NKG, qg = wave / NKG;   // this wave's score block
   const int64_t row0 = static_cast<int64_t>(blockIdx.x) * QT;
   const TX* x = static_cast<const TX*>(p.x);
 
   // One memory round trip: beta, the rows (past the end the last one repeats,
   // never stored) and the first key tiles.
   const ScalarHalves beta_bits = fetch_scalar(p.beta_ptr ? p.beta_ptr : p.x, p.beta_ptr ? p.beta_dtype : kF32, 0);
-  typename Elem<TX>::v8 xr[QPW][KS];
-#pragma unroll
-  for (int i = 0; i < QPW; ++i) {
+  typename Elem<TX>::v8 xr[KS];
+  const int own = qg * 16 + c;   // this lane's row of the score block
+  {
     const int64_t left = p.rows - 1 - row0;
-    const int at = (qg * QPW + i) * 16 + c;
-    const TX* src = x + (row0 + (at < left ? at : left)) * p.x_stride + 8 * g;
+    const TX* src = x + (row0 + (own < left ? own : left)) * p.x_stride + 8 * g;
 #pragma unroll
-    for (int kk = 0; kk < KS; ++kk) xr[i][kk] = load8(src + kk * 32);
+    for (int kk = 0; kk < KS; ++kk) xr[kk] = load8(src + kk * 32);
   }
   uint32_t koff[KCH];
 #pragma unroll
@@ -123,24 +120,21 @@ __global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams
   const float sign = beta < 0.f ? -1.f : 1.f;
   // With input normalization the unit row is rounded once to TK; otherwise
   // TK == TX and the raw row passes through unchanged.
-  k8 xf[QPW][KS];
+  k8 xf[KS];
+  float ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < QPW; ++i) {
-    float ss = 0.f;
+  for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
-    for (int kk = 0; kk < KS; ++kk)
+    for (int e = 0; e < 8; ++e) {
+      const float v = static_cast<float>(xr[kk][e]);
+      ss += v * v;
+    }
+  ss = group_sum(ss);
+  const float inv = sign * ((p.flags & kRouteNormalizeInput) ? 1.f / fmaxf(sqrtf(ss), p.eps) : 1.f);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float v = static_cast<float>(xr[i][kk][e]);
-        ss += v * v;
-      }
-    ss = group_sum(ss);
-    const float inv = sign * ((p.flags & kRouteNormalizeInput) ? 1.f / fmaxf(sqrtf(ss), p.eps) : 1.f);
+  for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
-    for (int kk = 0; kk < KS; ++kk)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) xf[i][kk][e] = static_cast<TK>(static_cast<float>(xr[i][kk][e]) * inv);
-  }
+    for (int e = 0; e < 8; ++e) xf[kk][e] = static_cast<TK>(static_cast<float>(xr[kk][e]) * inv);
 
   const _Float16* vbase = p.value + 32 * (wave * FB * 16) + c * 32 + g * 8;
   f16x8 vreg[KW][FB];
@@ -155,27 +149,23 @@ __global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams
   int kfrag[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) kfrag[k] = KTile::base(c, g, k) + kg * KTile::ROW_BLOCK;
-  // Logits of tile t: lane (c, g) element e of block i is atom atom_of(t) + e
-  // for row 16 (qg QPW + i) + c.
-  auto logits = [&](int t, f32x4 (&st)[QPW]) {
+  // Logits of tile t: lane (c, g) element e is atom atom_of(t) + e for row own.
+  auto logits = [&](int t) {
     const char* tile = lds + (t & 1) * KTile::BYTES;
+    f32x4 st = zero4();
 #pragma unroll
-    for (int i = 0; i < QPW; ++i) st[i] = zero4();
-#pragma unroll
-    for (int kk = 0; kk < KS; ++kk) {
-      const k8 a = lds_v8<TK>(tile + kfrag[kk & 3] + 256 * (kk >> 2));
-#pragma unroll
-      for (int i = 0; i < QPW; ++i) st[i] = Elem<TK>::mma(a, xf[i][kk], st[i]);
-    }
+    for (int kk = 0; kk < KS; ++kk)
+      st = Elem<TK>::mma(lds_v8<TK>(tile + kfrag[kk & 3] + 256 * (kk >> 2)), xf[kk], st);
     // Four fragments stay in flight ahead of their MFMAs.
     constexpr int AHEAD = 4;
     __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
 #pragma unroll
     for (int n = 0; n < KS - AHEAD; ++n) {
-      __builtin_amdgcn_sched_group_barrier(0x008, QPW, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, AHEAD * QPW, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
+    return st;
   };
   auto atom_of = [&](int t) { return t * KT + 32 * (kg >> 1) + 8 * g + 4 * (kg & 1); };
 
@@ -184,39 +174,26 @@ __global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams
   // each row's maximum from a pass over the atoms.  The largest weight is at
   // most 2^kRouteP16Lift; the factor cancels in the division by the row sum.
   const bool fixed = (p.flags & kRouteNormalizeInput) && (p.flags & kRouteUnitKeys) && 2.f * scale <= 2.f * kRouteP16Lift;
-  float ref[QPW];
-#pragma unroll
-  for (int i = 0; i < QPW; ++i) ref[i] = kRouteP16Lift - scale;
+  float ref = kRouteP16Lift - scale;
   if (!fixed) {
-    float mx[QPW];
-#pragma unroll
-    for (int i = 0; i < QPW; ++i) mx[i] = -INFINITY;
+    float mx = -INFINITY;
     for (int t = 0; t < n_tiles; ++t) {
       wait_vmem();
       lds_barrier();
       if (t > 0 && t + 1 < n_tiles) load_keys(t + 1);
-      f32x4 st[QPW];
-      logits(t, st);
+      const f32x4 st = logits(t);
 #pragma unroll
-      for (int i = 0; i < QPW; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (atom_of(t) + e < p.M) mx[i] = fmaxf(mx[i], st[i][e] * scale);
+      for (int e = 0; e < 4; ++e)
+        if (atom_of(t) + e < p.M) mx = fmaxf(mx, st[e] * scale);
     }
     float* xch = reinterpret_cast<float*>(lds + OFF_P);
-#pragma unroll
-    for (int i = 0; i < QPW; ++i) {
-      const float m = group_max(mx[i]);
-      if (g == 0) xch[kg * QT + (qg * QPW + i) * 16 + c] = m;
-    }
+    mx = group_max(mx);
+    if (g == 0) xch[kg * QT + own] = mx;
     lds_barrier();
+    float m = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < QPW; ++i) {
-      float m = -INFINITY;
-#pragma unroll
-      for (int w = 0; w < NKG; ++w) m = fmaxf(m, xch[w * QT + (qg * QPW + i) * 16 + c]);
-      ref[i] = m == -INFINITY ? 0.f : kRouteP16Lift - m;
-    }
+    for (int w = 0; w < NKG; ++w) m = fmaxf(m, xch[w * QT + own]);
+    ref = m == -INFINITY ? 0.f : kRouteP16Lift - m;
     // The pipeline restarts at the first tile (every wave is past its reads of
     // both key buffers; the barrier below is past the exchange's).
     wait_vmem();
@@ -230,34 +207,24 @@ __global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams
   for (int f = 0; f < FB; ++f)
 #pragma unroll
     for (int i = 0; i < QB; ++i) acc[f][i] = zero4();
-  float l_part[QPW];
-#pragma unroll
-  for (int i = 0; i < QPW; ++i) l_part[i] = 0.f;
+  float l_part = 0.f;
 
   // Logits of tile t, turned into weights in its P buffer.
   auto weights = [&](int t) {
     char* dst = lds + OFF_P + (t & 1) * PBYTES + (kg >> 1) * QB * 1024 + (kg & 1) * 8;
-    f32x4 pr[QPW];
-    logits(t, pr);
+    f32x4 pr = logits(t);
 #pragma unroll
-    for (int i = 0; i < QPW; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) pr[i][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(pr[i][e], scale, ref[i]));
+    for (int e = 0; e < 4; ++e) pr[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(pr[e], scale, ref));
     if ((t + 1) * KT > p.M) {   // padding atoms weigh nothing
 #pragma unroll
-      for (int i = 0; i < QPW; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (atom_of(t) + e >= p.M) pr[i][e] = 0.f;
+      for (int e = 0; e < 4; ++e)
+        if (atom_of(t) + e >= p.M) pr[e] = 0.f;
     }
+    l_part += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+    f16x4 h;
 #pragma unroll
-    for (int i = 0; i < QPW; ++i) {
-      l_part[i] += (pr[i][0] + pr[i][1]) + (pr[i][2] + pr[i][3]);
-      f16x4 h;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) h[e] = static_cast<_Float16>(pr[i][e]);
-      *reinterpret_cast<f16x4*>(dst + ((qg * QPW + i) * 64 + lane) * 16) = h;
-    }
+    for (int e = 0; e < 4; ++e) h[e] = static_cast<_Float16>(pr[e]);
+    *reinterpret_cast<f16x4*>(dst + (qg * 64 + lane) * 16) = h;
   };
   // O^T += Dv(t) P^T(t).
   auto multiply = [&](int t) {
@@ -308,11 +275,8 @@ __global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams
   float* xl = reinterpret_cast<float*>(lds + OFF_P);
   float* xn = reinterpret_cast<float*>(lds + OFF_P + PBYTES);
   lds_barrier();
-#pragma unroll
-  for (int i = 0; i < QPW; ++i) {
-    const float l = group_sum(l_part[i]);
-    if (g == 0) xl[kg * QT + (qg * QPW + i) * 16 + c] = l;
-  }
+  l_part = group_sum(l_part);
+  if (g == 0) xl[kg * QT + own] = l_part;
   lds_barrier();
   float w[QB];
 #pragma unroll
@@ -362,7 +326,7 @@ __global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams
 
 namespace {
 
-template <typename TX, typename TK, typename TO, int R, int QT, int KT, int QPW>
+template <typename TX, typename TK, typename TO, int R, int QT, int KT>
 void launch_k(const RouteArgs& a, hipStream_t s) {
   static_assert(kAtomPad % KT == 0, "the bank is padded to whole tiles");
   RouteTileParams p{};
@@ -380,7 +344,7 @@ void launch_k(const RouteArgs& a, hipStream_t s) {
   p.flags = a.flags;
   p.out = a.out;
   p.out_stride = a.out_stride;
-  hipLaunchKernelGGL((route_tile_kernel<TX, TK, TO, R, QT, KT, QPW>), dim3(static_cast<unsigned>((a.rows + QT - 1) / QT)),
+  hipLaunchKernelGGL((route_tile_kernel<TX, TK, TO, R, QT, KT>), dim3(static_cast<unsigned>((a.rows + QT - 1) / QT)),
                      dim3(kWaves * 64), 0, s, p);
 }
 
@@ -392,11 +356,11 @@ constexpr int64_t kTileCUs = 256;
 template <typename TX, typename TK, typename TO>
 void launch_t(const RouteArgs& a, hipStream_t s) {
   if (a.R == 256) {
-    launch_k<TX, TK, TO, 256, 32, 64, 1>(a, s);
+    launch_k<TX, TK, TO, 256, 32, 64>(a, s);
   } else if ((a.rows + 31) / 32 > kTileCUs) {
-    launch_k<TX, TK, TO, 512, 64, 32, 1>(a, s);
+    launch_k<TX, TK, TO, 512, 64, 32>(a, s);
   } else {
-    launch_k<TX, TK, TO, 512, 32, 64, 1>(a, s);
+    launch_k<TX, TK, TO, 512, 32, 64>(a, s);
   }
 }
 
