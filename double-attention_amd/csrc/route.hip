@@ -516,8 +516,8 @@ static void launch_route_t(const RouteArgs& a, hipStream_t s) {
 void launch_dictionary_route(const RouteArgs& a, hipStream_t stream) {
   if (a.rows == 0) return;
   // Eight-wave workgroups for 512-wide rows, and for 256-wide rows that do not
-  // give every CU 64 of them (M = 512: 12000 rows 19.3 us against 26.3 here,
-  // 8192 rows 12.6 / 14.8, but 16384 rows 19.8 / 17.6).
+  // give every CU 64 of them (M = 512: 12000 rows 19.8 us against 25.6 here,
+  // 8192 rows 12.2 / 13.8, but 16384 rows 19.8 / 17.6).
   if (!(a.flags & kRouteVariants) && (a.R == 512 || (a.R == 256 && (a.rows + kRouteRows - 1) / kRouteRows < kRouteCUs))) {
     launch_route_tile(a, stream);
     return;

@@ -16,16 +16,19 @@
 // waves share a SIMD.  What bounds it: the chain of one step (key loads, key
 // fragments, exponentials, the P exchange, the barrier), about 3000 clocks for
 // 1024 of MFMA work at R = 512.  A third key buffer with loads a whole step
-// ahead was slower (80 us against 71 at 16384 rows x 1536 atoms).  Measured (us,
-// bf16 rows, beta 8, against route.hip's kernel): R = 512 with 1536 atoms 192 rows 39 /
-// 67, 8192 rows 45 / 70, 16384 rows 62 / 74, 65536 rows 246 / 279; R = 256 with
-// 512 atoms 192 rows 11.0 / 12.9, 8192 rows 12.6 / 14.8, 12000 rows 19.3 / 26.3.
-// Where beta is too large for the fixed reference the extra pass over the
-// logits takes back the gain at 1536 atoms (beta 20: R = 256 8192 rows 33.9 / 32.6,
-// R = 512 8192 rows 61 / 86, 16384 rows 89 / 88).
-// Step t multiplies P(t) while it forms the weights of t+1, one barrier per
-// step; key tiles reach a two-buffer LDS ring by global->LDS DMA issued at the
-// start of a step.
+// ahead was slower (80 us against 71 at 16384 rows x 1536 atoms).
+// Step t multiplies P(t), turns the logits of t+1 into weights and forms those
+// of t+2, one barrier per step; key tiles reach a two-buffer LDS ring by
+// global->LDS DMA issued at the start of a step.  With the logits a tile ahead,
+// the row maxima that a beta above 9.7 needs are exchanged by that barrier, and
+// the sums are scaled as a maximum moves: no pass of its own over the atoms, which
+// cost 40 % (R = 512, 1536 atoms, 8192 rows 63 us, now 49).  Fixed-reference
+// calls pay 1 to 3 % for it, a barrier before the first step.
+// Measured (us, bf16 rows, against route.hip's kernel): beta 8, R = 512 with 1536
+// atoms 192 rows 40 / 68, 8192 rows 45 / 69, 12000 rows 60 / 70, 16384 rows 63 / 71,
+// 32768 rows 124 / 140; R = 256 with 512 atoms 192 rows 11.3 / 12.9, 8192 rows 12.2 /
+// 13.8, 12000 rows 19.8 / 25.6.  Beta 12: R = 512 with 1536 atoms 8192 rows 49 / 86,
+// 16384 rows 77 / 86; R = 256 with 1536 atoms 8192 rows 28.9 / 30.7, with 4096 atoms 74 / 77.
 #include <type_traits>
 
 #include "da_common.h"
@@ -55,7 +58,8 @@ struct RouteTileParams {
 }  // namespace
 
 template <typename TX, typename TK, typename TO, int R, int QT, int KT>
-__global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams p) {
+// 256-wide rows keep two workgroups per CU.
+__global__ __launch_bounds__(kWaves * 64, R == 256 ? 4 : 2) void route_tile_kernel(RouteTileParams p) {
   // x and out may alias (in-place routing): the workgroup has read its rows
   // into VGPRs, a barrier or more before any of its waves writes one.
   typedef typename Elem<TK>::v8 k8;
@@ -69,9 +73,11 @@ __global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams
   constexpr int KCH = KTile::LOADS / kWaves;   // wave loads of a key tile per wave
   constexpr int PBYTES = KW * QB * 1024;
   constexpr int OFF_P = 2 * KTile::BYTES;
-  // The P buffers also take the exchanges of row maxima, sums and norms.
+  // The P buffers also take the exchanges of row sums and norms; the maxima of
+  // two tiles (a row's from every wave along the atoms) follow them.
   static_assert(NKG * QT * 4 <= PBYTES && kWaves * QT * 4 <= PBYTES, "the exchanges fit a P buffer each");
-  __shared__ __attribute__((aligned(1024))) char lds[OFF_P + 2 * PBYTES];
+  constexpr int OFF_M = OFF_P + 2 * PBYTES, MBYTES = QT * NKG * 4;
+  __shared__ __attribute__((aligned(1024))) char lds[OFF_M + 2 * MBYTES];
 
   const int lane = lane_id();
   const int c = lane & 15, g = lane >> 4;
@@ -171,36 +177,10 @@ __global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams
 
   // The reference of the exponents: fixed where unit rows and unit atoms bound
   // every logit by 1 and all weights then stay in fp16's normal range, else
-  // each row's maximum from a pass over the atoms.  The largest weight is at
-  // most 2^kRouteP16Lift; the factor cancels in the division by the row sum.
+  // each row's maximum so far.  The largest weight is at most 2^kRouteP16Lift;
+  // the factor cancels in the division by the row sum.
   const bool fixed = (p.flags & kRouteNormalizeInput) && (p.flags & kRouteUnitKeys) && 2.f * scale <= 2.f * kRouteP16Lift;
-  float ref = kRouteP16Lift - scale;
-  if (!fixed) {
-    float mx = -INFINITY;
-    for (int t = 0; t < n_tiles; ++t) {
-      wait_vmem();
-      lds_barrier();
-      if (t > 0 && t + 1 < n_tiles) load_keys(t + 1);
-      const f32x4 st = logits(t);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (atom_of(t) + e < p.M) mx = fmaxf(mx, st[e] * scale);
-    }
-    float* xch = reinterpret_cast<float*>(lds + OFF_P);
-    mx = group_max(mx);
-    if (g == 0) xch[kg * QT + own] = mx;
-    lds_barrier();
-    float m = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < NKG; ++w) m = fmaxf(m, xch[w * QT + own]);
-    ref = m == -INFINITY ? 0.f : kRouteP16Lift - m;
-    // The pipeline restarts at the first tile (every wave is past its reads of
-    // both key buffers; the barrier below is past the exchange's).
-    wait_vmem();
-    load_keys(0);
-    if (n_tiles > 1) load_keys(1);
-    wait_vmem();
-  }
+  float ref = fixed ? kRouteP16Lift - scale : 0.f;
 
   f32x4 acc[FB][QB];
 #pragma unroll
@@ -209,10 +189,9 @@ __global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams
     for (int i = 0; i < QB; ++i) acc[f][i] = zero4();
   float l_part = 0.f;
 
-  // Logits of tile t, turned into weights in its P buffer.
-  auto weights = [&](int t) {
+  // Logits pr of tile t, turned into weights in its P buffer.
+  auto weights = [&](int t, f32x4 pr) {
     char* dst = lds + OFF_P + (t & 1) * PBYTES + (kg >> 1) * QB * 1024 + (kg & 1) * 8;
-    f32x4 pr = logits(t);
 #pragma unroll
     for (int e = 0; e < 4; ++e) pr[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(pr[e], scale, ref));
     if ((t + 1) * KT > p.M) {   // padding atoms weigh nothing
@@ -250,19 +229,68 @@ __global__ __launch_bounds__(kWaves * 64) void route_tile_kernel(RouteTileParams
   lds_barrier();   // key tiles 0 and 1
   load_values(0);
   __builtin_amdgcn_sched_barrier(0);
-  weights(0);
-
-  // Step t finds P(t) and the keys of t + 1 in LDS; the key buffer of t and
-  // the P buffer of t - 1 are free.
+  // Logits run a tile ahead of their weights.  Without the fixed reference the
+  // waves along the atoms have so exchanged a tile's row maxima by the step's
+  // own barrier.
+  auto maxima = [&](int t, const f32x4& st) {
+    float mx = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (atom_of(t) + e < p.M) mx = fmaxf(mx, st[e] * scale);
+    mx = group_max(mx);
+    if (g == 0) *reinterpret_cast<float*>(lds + OFF_M + (t & 1) * MBYTES + (own * NKG + kg) * 4) = mx;
+  };
+  float m[QB];   // maxima of rows 16 i + c
+#pragma unroll
+  for (int i = 0; i < QB; ++i) m[i] = -INFINITY;
+  // Tile t's maxima move the reference; the sums so far are scaled to it.
+  auto advance = [&](int t) {
+#pragma unroll
+    for (int i = 0; i < QB; ++i) {
+      const float* row = reinterpret_cast<const float*>(lds + OFF_M + (t & 1) * MBYTES) + (16 * i + c) * NKG;
+      float mx = m[i];
+#pragma unroll
+      for (int w = 0; w < NKG; ++w) mx = fmaxf(mx, row[w]);
+      if (__ballot(mx > m[i])) {
+        const float by = mx > m[i] ? __builtin_amdgcn_exp2f(m[i] - mx) : 1.f;
+        m[i] = mx;
+#pragma unroll
+        for (int f = 0; f < FB; ++f) acc[f][i] *= by;
+        if (i == qg) {
+          ref = kRouteP16Lift - mx;
+          l_part *= by;
+        }
+      }
+    }
+  };
+  f32x4 st = logits(0);
+  if (!fixed) maxima(0, st);
+  lds_barrier();   // the maxima of tile 0; its key buffer is free
+  if (n_tiles > 2) load_keys(2);
+  __builtin_amdgcn_sched_barrier(0);
+  if (!fixed) advance(0);
+  weights(0, st);
+  if (n_tiles > 1) {
+    st = logits(1);
+    if (!fixed) maxima(1, st);
+  }
+  // Step t finds P(t), the maxima of t + 1 and the keys of t + 2 in LDS; the
+  // key buffer of t + 1 and the P buffer of t - 1 are free.
+  wait_vmem();
   for (int t = 0; t + 1 < n_tiles; ++t) {
     lds_barrier();
-    if (t + 2 < n_tiles) load_keys(t + 2);
+    if (t + 3 < n_tiles) load_keys(t + 3);
     __builtin_amdgcn_sched_barrier(0);
     multiply(t);
     wait_vmem();
     load_values(t + 1);
     __builtin_amdgcn_sched_barrier(0);
-    weights(t + 1);
+    if (!fixed) advance(t + 1);
+    weights(t + 1, st);
+    if (t + 2 < n_tiles) {
+      st = logits(t + 2);
+      if (!fixed) maxima(t + 2, st);
+    }
     __builtin_amdgcn_sched_barrier(0);
   }
   lds_barrier();
@@ -350,7 +378,8 @@ void launch_k(const RouteArgs& a, hipStream_t s) {
 
 // 512-wide rows: 64 rows per workgroup halve the reads of the dictionary, 32
 // spread fewer rows over twice the CUs (1536 atoms: 8192 rows 45 us in one
-// round of 32-row workgroups; in two rounds, 12000 rows take 83).
+// round of 32-row workgroups; 12000 rows 60 us in one round of 64-row ones, and
+// 83 in two rounds of 32-row ones).
 constexpr int64_t kTileCUs = 256;
 
 template <typename TX, typename TK, typename TO>
