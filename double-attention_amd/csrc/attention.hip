@@ -1303,8 +1303,8 @@ static int64_t host_all_tiles(int64_t n_qt, int64_t qtile, int64_t length, bool 
   return qtile / kKeyTile * (n_qt - 1) * n_qt / 2 + host_key_tiles(n_qt - 1, qtile, length, true);
 }
 
-// MI355X: 256 CUs of 160 KiB LDS; every attention variant holds more than 256
-// registers per lane, so a SIMD runs one wave.
+// MI355X: 256 CUs of 160 KiB LDS; every variant of this kernel holds more than
+// 256 registers per lane, so a SIMD runs one wave.
 constexpr int64_t kCUs = 256;
 constexpr int64_t kLdsBytes = 160 * 1024;
 

@@ -255,8 +255,11 @@ int da_dictionary_route_backward_rows(const float* logits, const float* grad_wei
  *   DA_ATTN_MIX: out(b, t) = sum_s alpha_s O_s(b, t), alpha = softmax(mix_logits)
  *     (uniform 1/maps if mix_logits is NULL); else O_s(b, t) goes to
  *     out + b*out_stride_b + t*out_stride_t + s*out_stride_s.
- *   workspace: NULL, or >= da_attention_workspace_bytes(...) bytes, 256-byte
- *     aligned (scratch for split key ranges; see below).
+ *   workspace: NULL, or scratch for split key ranges, 256-byte aligned, of
+ *     workspace_bytes bytes.  da_attention_workspace_bytes(...) always suffice.
+ *     Less is taken as long as it holds the general kernel's own split, which
+ *     then runs the call also where the long-sequence kernel would be faster
+ *     (DA_ERR_WORKSPACE below that).  The two round differently.
  *   score_bound: 0, or an upper bound on |q . k| over all raw query/key rows
  *     (1 for L2-normalized rows).  With a bound, maps whose scaled bound fits
  *     the probability type skip the online-softmax rescaling (bf16 V only).
@@ -277,9 +280,11 @@ int da_routed_attention(const void* query, const void* key, int64_t stride_b, in
                         int64_t out_stride_t, int64_t out_stride_s, void* workspace,
                         int64_t workspace_bytes, da_stream_t stream);
 
-/* Scratch bytes da_routed_attention can use (0 if it needs none): fp32
- * partials of long causal key ranges split over workgroups and merged by a
- * second kernel.  Passing a NULL workspace is always allowed (no splitting). */
+/* Scratch bytes da_routed_attention can use (0 if it needs none): pieces of
+ * long key ranges, causal or not, split over workgroups and merged by a second
+ * kernel.  The pieces are fp32, or in the value dtype where the general kernel
+ * splits a call with a 16-bit output.  Passing a NULL workspace is always
+ * allowed (no splitting). */
 int64_t da_attention_workspace_bytes(int64_t batch, int64_t maps, int64_t length, int64_t score_dim,
                                      int64_t value_dim, int flags);
 
@@ -515,7 +520,7 @@ typedef struct da_sda_forward_args {
   int dtype;                /* activation / weight dtype: DA_F16 or DA_BF16 */
   float eps;
   int flags;                /* DA_SDA_* */
-  void* workspace;          /* da_sda_workspace_bytes(...) bytes, 256-byte aligned */
+  void* workspace;          /* 256-byte aligned; da_sda_workspace_bytes(...) bytes always suffice */
   int64_t workspace_bytes;
   void* out;                /* [batch, length, model_dim] */
   /* Optional: the raw bank (da_dictionary_normalize's raw_key / raw_value /
@@ -540,8 +545,10 @@ typedef struct da_sda_forward_args {
  *   routed [tokens, 2*qk_width]   Q/K projections, routed in place (fp16 out)
  *   value_t [batch, padded_length/32, model_dim, 32]  (32-token tiles)
  *   mixed  [tokens, model_dim or maps*model_dim] (only with an output projection)
- *   then, with one outer map, fp32 partial results of the attention over
- *   chunks of long causal key ranges (merged by a second kernel). */
+ *   then, with one outer map, the scratch of da_routed_attention for long key
+ *   ranges.  A workspace that holds only the general attention kernel's share of
+ *   it is accepted too (DA_ERR_WORKSPACE below that): the call then runs that
+ *   kernel where the long-sequence one would need more. */
 int64_t da_sda_workspace_bytes(int64_t batch, int64_t length, int64_t model_dim,
                                int64_t qk_width, int64_t outer_maps, int concat,
                                int has_output_projection);
@@ -560,7 +567,9 @@ int da_shared_dictionary_attention_forward(const da_sda_forward_args* args, da_s
  * until the process ends), found once per device on its first call there;
  * the call uses the array of the device `stream` launches on (the current
  * device for the null stream).
- * Problems whose da_sda_workspace_bytes exceed it fail with DA_ERR_WORKSPACE.
+ * A problem that does not fit it fails with DA_ERR_WORKSPACE; one that fits only
+ * with the general attention kernel's scratch runs that kernel, and then differs
+ * in rounding from a call with a full workspace.
  * The call itself allocates nothing.  Every call on one GPU shares that GPU's
  * array, which keeps the last call's contents: calls that overlap on one GPU
  * (other streams, other threads) race, so serialize them.  The caller still
