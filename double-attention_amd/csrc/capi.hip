@@ -747,7 +747,6 @@ static int64_t sda_least_bytes(int64_t batch, int64_t length, int64_t model_dim,
 
 int64_t da_sda_workspace_bytes(int64_t batch, int64_t length, int64_t model_dim, int64_t qk_width,
                                int64_t outer_maps, int concat, int has_output_projection) {
-  if (outer_maps < 1) return 0;
   return da_sda_workspace_offset(batch, length, model_dim, qk_width, 2) +
          sda_mixed_bytes(batch * length, model_dim, outer_maps, concat != 0, has_output_projection != 0) +
          attention_scratch_bytes(batch, length, model_dim, qk_width, outer_maps);

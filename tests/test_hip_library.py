@@ -43,6 +43,8 @@ def test_abi_version_and_helpers() -> None:
     assert partials > 0 and partials % 256 == 0
     assert h.da_sda_workspace_bytes(1, 8192, 512, 256, 4, 0, 1) == base_c5
     assert h.da_sda_workspace_offset(8, 512, 512, 256, 1) == 4096 * 512 * 2
+    # Without a map there is no scratch of the outer attention.
+    assert h.da_sda_workspace_bytes(8, 512, 512, 256, 0, 0, 1) == 3 * 4096 * 512 * 2
 
 
 def _fake(addr: int = 1 << 20) -> int:
